@@ -82,8 +82,10 @@ __global__ __launch_bounds__(256) void linear_rows_mfma_kernel(RowsArgs p) {
       }
     }
     // short chains on the matrix unit, added up by rounding additions: long ones round worse (router logits of 8 rows, K = 1536: relative error
-    // 1.3e-7 in one chain a wave, 7e-8 so)
+    // 1.3e-7 in one chain a wave, 7e-8 so).  The U pieces of a turn are added to each other first (K = 17920, 2 rows: 1.67e-7 one by one,
+    // 1.06e-7 so)
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4_t turn[NT][MT];
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -95,15 +97,17 @@ __global__ __launch_bounds__(256) void linear_rows_mfma_kernel(RowsArgs p) {
 #pragma unroll
             for (int x = 0; x < 2; ++x)
               t[x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wv[u][j][x]), __builtin_bit_cast(bf16x8_t, av[u][i][x]), zero, 0, 0, 0);
-            acc[j][i] += t[0] + t[1];
+            t[0] += t[1];
           } else {
 #pragma unroll
             for (int y = 0; y < 16; ++y) {
               const unsigned q = wv[u][j][y / 8][y % 8 / 2], z = av[u][i][y / 4][y % 4];
               t[y % 4] = __builtin_amdgcn_mfma_f32_16x16x4f32(y & 1 ? bf_hi(q) : bf_lo(q), __builtin_bit_cast(float, z), t[y % 4], 0, 0, 0);
             }
-            acc[j][i] += (t[0] + t[1]) + (t[2] + t[3]);
+            t[0] = (t[0] + t[1]) + (t[2] + t[3]);
           }
+          turn[j][i] = u ? turn[j][i] + t[0] : t[0];
+          if (u == U - 1) acc[j][i] += turn[j][i];
         }
   }
 #pragma unroll
@@ -150,11 +154,13 @@ VLM_INTERNAL int vlm_linear_rows_mfma_try(const void* A, const void* W, void* C,
                                           int batch, long sA, long sW, long sC, int accumulate, void* stream) {
   // where the line lies: wider outputs fill the chip with whole tiles (9000 x 3584, 8 rows: 17.7 us on the GEMM's, 25.7 here), a longer K is better split
   // over workgroups (1536 x 8960, 16 rows: 12.6 and 15.2); many narrow maps of up to 8 rows are cheap here (28 of [512, 128]: 12.9 -> 4.6)
+  // fp32 sums onto a stream keep the long K here up to 8 rows: the split form hands over bf16 (1536 x 21696, 2 / 4 / 8 rows: 26 / 26 / 32; vlm_linear_rows_bf16w
+  // 48 / 76 / 140)
   const int va = a_f32 ? 4 : 8;
   // more rows over few columns, as blocks of 16: router logits [8, 1536] of 2048 rows 29 -> 7.5 us
   if (M > 32 ? N > 64 || batch > 1 || M > 65535 * 16 : false) return -1;
   const bool fits = (long)N * batch <= 8192 || (M <= 8 && (long)N * batch * K <= 4 << 20);
-  if (!fits || K > 4096 || K % 8 || lda % va || sA % va || ldw % 8 || sW % 8 || (((uintptr_t)A | (uintptr_t)W) & 15)) return -1;
+  if (!fits || (K > 4096 && !(accumulate && M <= 8)) || K % 8 || lda % va || sA % va || ldw % 8 || sW % 8 || (((uintptr_t)A | (uintptr_t)W) & 15)) return -1;
   const RowsArgs a{A, (const bf16_t*)W, C, M, N, K, 0, accumulate, lda, ldw, ldc, sA, sW, sC};
   hipStream_t st = (hipStream_t)stream;
   if (a_f32) c_f32 ? launch_rows<float, float>(a, batch, st) : launch_rows<float, bf16_t>(a, batch, st);

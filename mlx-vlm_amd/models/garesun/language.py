@@ -219,12 +219,12 @@ class LanguageModel(RaggedLanguageModel):
                 ops.moe_relu2_gate(col("up"), gate, ns.E, ns.ff, ns.sff, cat[:, ns.koff["ff"]:])
             if grouped:
                 pass
-            elif T == torch.bfloat16 and (Tn > self.STREAM_ROWS or (Tn > 1 and cat.shape[1] > 4096)):
+            elif T == torch.bfloat16 and Tn > self.STREAM_ROWS:
                 y = self._linear(cat, ns.wout)
                 ops.stream_add_(x, y)
                 keep.append(y)
             elif few:
-                self._linear(cat, ns.wout, out=x, accumulate=True)      # (unchosen experts: zero activations, weights not read)
+                self._linear(cat, ns.wout, out=x, accumulate=True)      # (fp32 sums straight onto the stream)
             else:
                 ops.linear_any(cat, ns.wout, out=x, accumulate=True)
             if cfg.side_dim:

@@ -153,6 +153,11 @@ class RaggedLanguageModel:
         # [1536, 1536] 4.7 / 5.0 / 5.4, streaming 5.6 / 9.0, GEMM 7.5; [4616, 1536] 6.0 / 6.2 / 6.7, streaming 7.9 / 12.4, GEMM 8.5)
         if mfma and 3 <= M <= 32 and N <= 8192 and K <= 4096 and skip is None:
             return ops.linear_any(a, w, out=out, out_dtype=out_dtype, accumulate=accumulate)
+        # a long K summed in fp32 onto the stream likewise, up to 8 rows ([1536, 17920] with the columns of four or five of eight experts, 2 / 3 / 4 rows:
+        # 21 / 22 / 22, streaming, which leaves out weights that meet zeros alone, 20 / 48 / 59; [1536, 21696] of nine 26 / 26 / 26, streaming 48 / 64 / 76:
+        # past 20480 two rows no longer fit its LDS)
+        if mfma and accumulate and K > 4096 and N <= 8192 and (3 <= M <= 8 or (M == 2 and K > 20480)) and skip is None:
+            return ops.linear_any(a, w, out=out, out_dtype=out_dtype, accumulate=accumulate)
         # a long K is split over workgroups, in a capture too ([1536, 17920], 2 / 4 / 8 rows: 16.6 / 16.7 / 17.2, streaming 21 / 71 / 114, one pass 66)
         if (mfma and not accumulate and want == torch.bfloat16 and (M > self.STREAM_ROWS or (M > 1 and K > 4096)) and N % 8 == 0
                 and (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0))):

@@ -584,6 +584,28 @@ def test_linear_any_few_rows_over_bf16_weights(M, N, K, batch):
                 assert over.max() <= 0, (ta, tc, add)
 
 
+@pytest.mark.parametrize("experts", [6, 36])
+@pytest.mark.parametrize("rows", [1, 2, 3, 4])
+def test_steps_of_few_rows_sum_onto_the_stream_in_fp32(tmp_path, rows, experts):
+    """output projection of 1 to 4 decode rows over [mixer | experts] wider than 4096 and wider than 20480: the stream after a layer is the stream before it plus the
+    float64 product of the layer's bf16 rows, within the roundings of fp32 sums (a bf16 row on the way would be off by 2^-9)"""
+    cfg = H.config([H.layer("retention", ff=600, shared_ff=600, experts=experts) for _ in range(2)], side=0)
+    lm = _load(tmp_path, cfg, H.weights(cfg), "bfloat16")
+    lm = getattr(lm, "language_model", lm)
+    ns, seen, linear = lm._L[1], [], lm._linear
+    lm._linear = lambda a, w, **kw: (seen.append(a.double()) if w is ns.wout else None, linear(a, w, **kw))[1]
+    lm._trace = []
+    caches = [lm.make_cache() for _ in range(rows)]
+    lm.step([(c[0]._seq, _ids(1, cfg["vocab"], 5 + i)) for i, c in enumerate(caches)], want="all")
+    before, after = (x.double() for x in lm._trace)
+    assert len(seen) == 1 and seen[0].shape == (rows, ns.wout.shape[1])
+    added = seen[0] @ ns.wout.double().T
+    # at most K / 256 + 12 roundings of partial sums below sum |a w|, and one of the stream
+    bound = seen[0].abs() @ ns.wout.double().abs().T * ((ns.wout.shape[1] / 256 + 12) * 2.0 ** -24) + after.abs() * 2.0 ** -24
+    assert ((after - before - added).abs() <= bound).all()
+    assert (after - before - added).norm() < 2.0 ** -20 * added.norm()
+
+
 @pytest.mark.parametrize("M,N,K", [(2, 1536, 8960), (8, 1536, 17920), (33, 264, 4160), (64, 3584, 4352)])
 def test_gemm_rows_splits_a_long_k_in_a_capture_too(M, N, K):
     from mlx_vlm_amd import ops
