@@ -158,8 +158,12 @@ class RaggedLanguageModel:
         # past 20480 two rows no longer fit its LDS)
         if mfma and accumulate and K > 4096 and N <= 8192 and (3 <= M <= 8 or (M == 2 and K > 20480)) and skip is None:
             return ops.linear_any(a, w, out=out, out_dtype=out_dtype, accumulate=accumulate)
-        # a long K is split over workgroups, in a capture too ([1536, 17920], 2 / 4 / 8 rows: 16.6 / 16.7 / 17.2, streaming 21 / 71 / 114, one pass 66)
-        if (mfma and not accumulate and want == torch.bfloat16 and (M > self.STREAM_ROWS or (M > 1 and K > 4096)) and N % 8 == 0
+        # a long K is split over workgroups, in a capture too ([1536, 17920], 2 / 3 / 4 / 8 rows: 17 / 17 / 17 / 17; streaming 22 / 64 / 72 / 114, and over the zeros
+        # of unchosen experts 20 / 47 / 58 / 100; one pass 66).  Two rows from K = 8192 and below 16384 columns ([1536, 4736] 9.9, streaming 7.9; [1536, 6720] 10.5 and
+        # 10.0; [1536, 8960] 11.7 and 12.2; [35840, 4608] 70 and 56); three on a par at [4608, 4608] (15.5 and 15.1).  With `skip` up to STREAM_ROWS rows
+        # stay with the form that leaves columns out ([35840, 4608], two of eight experts a row, 2 / 3 / 4 rows 37 / 50 / 69, the GEMM 70 / 69 / 70)
+        split = K > 4096 and K % 64 == 0 and skip is None and (M > 2 or (M == 2 and K >= 8192 and N < 16384))
+        if (mfma and not accumulate and want == torch.bfloat16 and (M > self.STREAM_ROWS or split) and N % 8 == 0
                 and (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0))):
             return ops.gemm_rows(a, w, out=out) if M <= 64 and K > 4096 else ops.gemm(a, w, out=out)
         if M <= 8 and w.dtype == torch.bfloat16 and K % 8 == 0 and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0:

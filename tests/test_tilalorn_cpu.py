@@ -134,3 +134,23 @@ def test_oracle_router_keeps_the_best_groups_and_does_not_renormalise():
     assert torch.nonzero(w[0]).view(-1).tolist() == [0, 4, 5]                     # expert 2 scores higher than 4 but its group is out
     w = O.route(z, dict(experts=6, top=3, scale=1.0))
     assert torch.nonzero(w[0]).view(-1).tolist() == [0, 2, 5]
+
+
+@pytest.mark.parametrize("M,N,K,skip,route", [
+    (2, 4096, 4608, True, "linear_rows_bf16w"), (3, 4096, 4608, True, "linear_rows_bf16w"), (4, 4096, 4608, True, "linear_rows_bf16w"),      # the columns of experts are left out
+    (5, 4096, 4608, False, "gemm_rows"), (4, 4096, 4608, False, "gemm_rows"), (3, 4096, 4616, False, "linear_rows_bf16w"),             # (a K that is not split)
+    (2, 1536, 4736, False, "linear_rows_bf16w"), (2, 1536, 8960, False, "gemm_rows"), (2, 16384, 8960, False, "linear_rows_bf16w"), (1, 1536, 17920, False, "linear_rows_bf16w"),
+    (3, 1536, 1536, False, "linear_any"), (3, 1536, 1536, True, "linear_rows_bf16w"), (65, 1536, 4608, False, "gemm")])
+def test_products_of_few_rows_take_the_form_that_was_measured_for_them(monkeypatch, M, N, K, skip, route):
+    """up to STREAM_ROWS rows with an expert table keep the form that leaves columns out, whatever K"""
+    from mlx_vlm_amd import ops
+    from mlx_vlm_amd.models.ragged import RaggedLanguageModel
+
+    taken = []
+    for name in ("linear_any", "linear_rows_bf16w", "gemm", "gemm_rows"):
+        monkeypatch.setattr(ops, name, lambda a, w, _n=name, **kw: taken.append((_n, kw.get("skip_gate"))))
+    lm = RaggedLanguageModel.__new__(RaggedLanguageModel)
+    a, w = torch.empty(M, K, dtype=torch.bfloat16), torch.empty(N, K, dtype=torch.bfloat16)
+    gate = torch.ones(M, 2)
+    lm._linear(a, w, skip=dict(skip_gate=gate, skip_col0=0, E=2, ff=N // 2) if skip else None)
+    assert taken == [(route, gate if skip else None)]
