@@ -620,7 +620,7 @@ typedef struct vlm_recurrence_args {
   int row_norm;                         /* ABI v13, gated = 0: ONE RMS norm over all heads of the token instead of one per head */
   float* ws;                            /* ABI v13: workspace of the chunk-parallel form (gated = 0 / 1), or NULL */
   long ws_floats;                       /* its size: H * D * (Dv + gated) per chunk of 64 tokens (at least one, fewer chunks run in windows), and with
-                                           rotation 2 * H * D, with gated = 1 4 * H a token on top (less: token by token) */
+                                           rotation 2 * H * D, with gated = 1 4 * H a token on top (less, or gated = 1 with rotation: token by token) */
 } vlm_recurrence_args;
 int vlm_linear_recurrence(const vlm_recurrence_args* a, int nseg, int ntok, int dtype, void* stream);
 

@@ -455,7 +455,9 @@ int run_chunks(const vlm_recurrence_args& a, int nseg, int ntok, int max_len, hi
     float* ig = a.ws + 2 * (long)ntok * a.H;
     hipLaunchKernelGGL((gate_scan_kernel<T>), dim3(nseg, a.H), dim3(1024), 0, st, a, max_len, F, ig);
     VLM_CHECK_LAUNCH();
-    return run_windows<T, T, true>(a, GateRows{F, ig}, nseg, ntok, max_len, ws, left, st);
+    vlm_recurrence_args b = a;
+    b.q_act = 0;                                                         // (an activation of q belongs to the other recurrences)
+    return run_windows<T, T, true>(b, GateRows{F, ig}, nseg, ntok, max_len, ws, left, st);
   }
   if (a.rot_dims) {
     hipLaunchKernelGGL((chunk_rotate_kernel<T>), dim3(ntok, 2), dim3(256), 0, st, a, nseg, max_len, ntok, a.ws);

@@ -19,8 +19,8 @@
 // vlm_linear_recurrence writes the raw o (and n . q) in fp32; vlm_recurrence_finish then applies the denominator, the
 // per-head unit-RMS norm (row_norm: ONE norm over all heads of the token), an optional weight and the output gate (silu or sigmoid of a projection) into a T-typed row.
 //
-// With a workspace (ws) that holds one chunk, fixed-decay and exponentially gated segments of VLM_CHUNK_MIN tokens or more run chunk-parallel on
-// the matrix cores instead (chunk_recurrence.hip).
+// With a workspace (ws) that holds one chunk, fixed-decay and (unrotated) exponentially gated segments of VLM_CHUNK_MIN tokens or more run
+// chunk-parallel on the matrix cores instead (chunk_recurrence.hip).
 //
 // Work split: workgroup = (segment, head, tile of 64 state columns); lane c of part p holds rows [32 p, 32 p + 32) of column
 // c in registers.  Tokens are staged 4 / 8 / 16 at a time through LDS (q, k rotated and scaled on the way in).
@@ -238,7 +238,7 @@ int run(const vlm_recurrence_args& a, int nseg, int ntok, hipStream_t st) {
   dim3 grid(nseg, a.H, (C + CT - 1) / CT), block(P * CT);
   int max_len = 0x7fffffff;
   const int longest = ntok - nseg + 1;                   // no segment of the step is longer (every segment has a token)
-  if (!rowgate && a.ws && longest >= VLM_CHUNK_MIN && a.ws_floats - vlm_chunk_prep_floats(&a, ntok) >= (long)a.H * a.D * C) {
+  if (!rowgate && !(gated && a.rot_dims) && a.ws && longest >= VLM_CHUNK_MIN && a.ws_floats - vlm_chunk_prep_floats(&a, ntok) >= (long)a.H * a.D * C) {
     max_len = VLM_CHUNK_MIN - 1;
     const int rc = vlm_chunk_recurrence(&a, nseg, ntok, max_len, sizeof(T) == 4, st);
     if (rc) return rc;

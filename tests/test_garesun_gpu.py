@@ -236,6 +236,42 @@ def test_chunk_parallel_recurrences_against_the_token_by_token_kernel(gated, rot
     assert all(torch.equal(x, y) for x, y in zip(run(Hh * D * Dv), serial))         # no room behind the prepared rows: token by token
 
 
+@pytest.mark.parametrize("gated,rot,q_act,decays", [(1, 20, 0, None), (1, 0, 1, None), (1, 20, 1, None), (0, 0, 1, [0.9, 0.5]), (0, 20, 0, [0.9, 0.5])])
+def test_a_workspace_changes_no_recurrence(gated, rot, q_act, decays):
+    """every form of the call that is accepted, with a workspace and without: gated heads with rotated keys, and with the flag of an activation that gated heads
+    do not have.  Sums of another order: 2^-18 of the largest value"""
+    from mlx_vlm_amd import _lib, ops
+
+    g, T, Hh, D, Dv = torch.Generator().manual_seed(rot + q_act), 150, 2, 32, 24
+    C = Dv + gated
+    q, k = (torch.randn(T, Hh * D, generator=g).bfloat16().cuda() for _ in range(2))
+    v, gate = (torch.randn(T, Hh * Dv, generator=g).bfloat16().cuda() for _ in range(2))
+    pre = torch.randn(2, T, Hh, generator=g).bfloat16().cuda()
+    bias, decay = torch.ones(Hh).bfloat16().cuda(), torch.tensor(decays or [0.5] * Hh).cuda()
+    inv = torch.tensor([1e4 ** (-2 * i / 20) for i in range(10)]).cuda()
+    state0, m0 = torch.randn(2, Hh, D, C, generator=g), torch.randn(2, Hh, generator=g)
+    tab = torch.tensor([0, T, 1, 7], dtype=torch.int32).cuda()
+
+    def run(ws):
+        state, ms, mtok, mprev = state0.cuda(), m0.cuda(), torch.empty(T, Hh, device="cuda"), torch.empty(1, Hh, device="cuda")
+        raw, out = torch.empty(T, Hh, C, device="cuda"), torch.empty(T, Hh * Dv, dtype=torch.bfloat16, device="cuda")
+        a = _lib.RecurrenceArgs()
+        a.q, a.k, a.v, a.g, a.ldq, a.ldk, a.ldv, a.ldg, a.ldo = q.data_ptr(), k.data_ptr(), v.data_ptr(), gate.data_ptr(), Hh * D, Hh * D, Hh * Dv, Hh * Dv, Hh * Dv
+        a.qscale, a.kscale, a.eps, a.gate_act, a.gated, a.rot_dims, a.q_act, a.decay, a.inv_freq = 0.5, 0.25, 1e-5, 1, gated, rot, q_act, decay.data_ptr(), inv.data_ptr()
+        a.ipre, a.fpre, a.ldi, a.ldf, a.ib, a.fb, a.cap = pre[0].data_ptr(), pre[1].data_ptr(), Hh, Hh, bias.data_ptr(), bias.data_ptr(), 12.0
+        a.mstate, a.mtok, a.mprev = ms.data_ptr(), mtok.data_ptr(), mprev.data_ptr()
+        a.seg_start, a.seg_slot, a.seg_pos0 = tab.data_ptr(), tab[2:].data_ptr(), tab[3:].data_ptr()
+        a.state, a.raw, a.out, a.H, a.D, a.Dv = state.data_ptr(), raw.data_ptr(), out.data_ptr(), Hh, D, Dv
+        if ws is not None:
+            a.ws, a.ws_floats = ws.data_ptr(), ws.numel()
+        ops.linear_recurrence(a, 1, T, False)
+        torch.cuda.synchronize()
+        return raw.cpu().double(), state.cpu().double(), ms.cpu().double()
+
+    for got, want in zip(run(torch.empty(1 << 20, device="cuda")), run(None)):
+        assert (got - want).abs().max() <= want.abs().max() * 2.0 ** -18
+
+
 # ------------------------------------------------------------------------------------------------ schedules
 @pytest.fixture(scope="module")
 def mixed32(tmp_path_factory):
