@@ -41,8 +41,16 @@ constexpr int CH = VLM_CHUNK;
 
 __device__ __forceinline__ float silu_f(float x) { return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x)); }
 
-// a^n for n >= 0 (a >= 0), exact for n = 0 and a = 0
-__device__ __forceinline__ float powi(float l2a, int n) { return n == 0 ? 1.f : __builtin_amdgcn_exp2f(l2a * (float)n); }
+// a^n for n >= 0, exact for n = 0 and a = 0
+struct Power {
+  float l2;                      // log2 |a|
+  unsigned sign;                 // the sign bit of a
+};
+__device__ __forceinline__ Power power_of(float a) { return Power{__builtin_amdgcn_logf(fabsf(a)), __float_as_uint(a) & 0x80000000u}; }
+__device__ __forceinline__ float powi(Power a, int n) {
+  const float r = n == 0 ? 1.f : __builtin_amdgcn_exp2f(a.l2 * (float)n);
+  return __uint_as_float(__float_as_uint(r) ^ (n & 1 ? a.sign : 0u));
+}
 
 // N consecutive values of a row, the first `have` of which exist
 template <int N> __device__ __forceinline__ void row_vals(const bf16_t* p, int have, bool vec, float* f) {
@@ -108,7 +116,7 @@ __global__ __launch_bounds__(256) void chunk_update_kernel(vlm_recurrence_args p
   const T* v = (const T*)p.v + (long)h * Dv + v0;
   const bool kvec = ((uintptr_t)p.k % (4 * sizeof(TK))) == 0 && p.ldk % 4 == 0 && D % 4 == 0;
   const bool vvec = ((uintptr_t)p.v % (4 * sizeof(T))) == 0 && p.ldv % 4 == 0 && Dv % 4 == 0;
-  const float l2a = GATED ? 0.f : __builtin_amdgcn_logf(p.decay[h]);     // log2
+  const Power pw = power_of(GATED ? 0.f : p.decay[h]);
   double Fm = 0.;                                                        // (gated) F - m at the chunk's last token
   if constexpr (GATED) Fm = gr.F[(long)(t0 + n - 1) * p.H + h] - (double)p.mtok[(long)(t0 + n - 1) * p.H + h];
   float nacc[4] = {};                                                    // (gated) the normaliser's entries of this lane's rows
@@ -126,7 +134,7 @@ __global__ __launch_bounds__(256) void chunk_update_kernel(vlm_recurrence_args p
     row_vals<4>(k + tok * p.ldk, live ? D - d0 : 0, kvec, kv);
     row_vals<4>(v + tok * p.ldv, live ? Dv - v0 : 0, vvec, vv);
     float w = 0.f;
-    if (live) w = (GATED ? exp_d(Fm - gr.F[tok * p.H + h] + (double)gr.ig[tok * p.H + h]) : powi(l2a, n - 1 - j)) * p.kscale;
+    if (live) w = (GATED ? exp_d(Fm - gr.F[tok * p.H + h] + (double)gr.ig[tok * p.H + h]) : powi(pw, n - 1 - j)) * p.kscale;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       kv[i] = (p.k_act ? silu_f(kv[i]) : kv[i]) * w;
@@ -214,8 +222,8 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(vlm_recurrence_args p, 
     *S = s;
     return;
   }
-  const float a = p.decay[h], l2a = __builtin_amdgcn_logf(a);
-  const float full = powi(l2a, CH);
+  const Power pw = power_of(p.decay[h]);
+  const float full = powi(pw, CH);
   for (; c + 4 < hi; c += 4, w += 4 * HE) {                              // whole chunks, four loads in flight
     float u[4];
 #pragma unroll
@@ -229,7 +237,7 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(vlm_recurrence_args p, 
   for (; c < hi; ++c, w += HE) {
     const float u = *w;
     *w = s;
-    s = fmaf(c + 1 < chunks ? full : powi(l2a, len - c * CH), s, u);
+    s = fmaf(c + 1 < chunks ? full : powi(pw, len - c * CH), s, u);
   }
   *S = s;
 }
@@ -252,7 +260,7 @@ __global__ __launch_bounds__(256) void chunk_output_kernel(vlm_recurrence_args p
   const float* S0 = ws + ((long)blockIdx.x * p.H + h) * (long)D * (Dv + GATED);
   const float* S = S0 + vcol;
   const bool svec = Dv % 4 == 0 && (((uintptr_t)S0) & 15) == 0;
-  const float l2a = GATED ? 0.f : __builtin_amdgcn_logf(p.decay[h]);
+  const Power pw = power_of(GATED ? 0.f : p.decay[h]);
   const long ti = (long)(t0 + min(i, n - 1)) * p.H + h;
   double Fm = 0.;                                                        // (gated) F - m of this lane's query
   float nq = 0.f, mine = 0.f;                                            // (gated) normaliser . q: the chunk's start, its tokens
@@ -295,7 +303,7 @@ __global__ __launch_bounds__(256) void chunk_output_kernel(vlm_recurrence_args p
     const int first = p.seg_start[seg];
     ai = exp_d(Fm + (double)(t0 > first ? p.mtok[(long)(t0 - 1) * p.H + h] : p.mprev[(long)seg * p.H + h]));
   } else {
-    ai = powi(l2a, i + 1);
+    ai = powi(pw, i + 1);
   }
 #pragma unroll
   for (int b = 0; b < NB; ++b) acc[b] *= ai;
@@ -311,7 +319,7 @@ __global__ __launch_bounds__(256) void chunk_output_kernel(vlm_recurrence_args p
           const long tj = (long)(t0 + min(j, n - 1)) * p.H + h;
           pr = s[t][r] * exp_d(Fm - gr.F[tj] + (double)gr.ig[tj]);
         } else {
-          pr = s[t][r] * powi(l2a, i - j);
+          pr = s[t][r] * powi(pw, i - j);
         }
       }
       mine += pr;

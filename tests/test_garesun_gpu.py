@@ -236,10 +236,11 @@ def test_chunk_parallel_recurrences_against_the_token_by_token_kernel(gated, rot
     assert all(torch.equal(x, y) for x, y in zip(run(Hh * D * Dv), serial))         # no room behind the prepared rows: token by token
 
 
-@pytest.mark.parametrize("gated,rot,q_act,decays", [(1, 20, 0, None), (1, 0, 1, None), (1, 20, 1, None), (0, 0, 1, [0.9, 0.5]), (0, 20, 0, [0.9, 0.5])])
+@pytest.mark.parametrize("gated,rot,q_act,decays", [(1, 20, 0, None), (1, 0, 1, None), (1, 20, 1, None), (0, 0, 1, [0.9, 0.5]), (0, 20, 0, [0.9, 0.5]),
+                                                    (0, 20, 0, [-0.9, 0.0]), (0, 0, 0, [-0.97, 1.0])])
 def test_a_workspace_changes_no_recurrence(gated, rot, q_act, decays):
     """every form of the call that is accepted, with a workspace and without: gated heads with rotated keys, and with the flag of an activation that gated heads
-    do not have.  Sums of another order: 2^-18 of the largest value"""
+    do not have; decays of either sign, zero and one.  Sums of another order: 2^-18 of the largest value"""
     from mlx_vlm_amd import _lib, ops
 
     g, T, Hh, D, Dv = torch.Generator().manual_seed(rot + q_act), 150, 2, 32, 24
