@@ -131,7 +131,7 @@ class LanguageModel(RaggedLanguageModel):
     def _experts_grouped(self, ns, h):
         """whether a step's experts are evaluated pair by pair (the shared feed-forward as one more expert, which every token takes)"""
         return (h.numel() >= self.GROUPED_SIZE and ns.sff in (0, ns.ff)
-                and ops.moe_grouped_fits(h, ns.wproj[ns.off["up"]:], ns.wout[:, ns.koff["ff"]:], ns.ff))
+                and ops.moe_grouped_fits(h, ns.wproj[ns.off["up"]:], ns.wout[:, ns.koff["ff"]:], ns.ff, ns.E + (ns.sff > 0)))
 
     def _run(self, pl, logits_dtype=torch.float32):
         """Device side of a step: nothing here looks at host data that changes between two steps of the same shape, so a

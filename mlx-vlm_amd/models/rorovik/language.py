@@ -181,7 +181,7 @@ class LanguageModel(RaggedLanguageModel):
             few = Tn <= self.STREAM_ROWS and T != torch.float32       # decode rows over bf16 weights: weight-streaming projections
             route, ident = ops.moe_router_softmax(h, ns.router, ns.top, ns.identity, ns.corr)
             step = dict(pass_=ident, src=h) if ident is not None else {}
-            if Tn >= self.GROUPED_ROWS and ops.moe_grouped_fits(h, ns.wff, ns.down, ff):
+            if Tn >= self.GROUPED_ROWS and ops.moe_grouped_fits(h, ns.wff, ns.down, ff, ns.E):
                 y, slots = ops.moe_grouped_rows(h, ns.wff, ns.down, route, ns.top, ops.GLU_CLAMPED, ns.limit)
                 keep += [route, y, step]
                 return y, dict(step, slots=slots)

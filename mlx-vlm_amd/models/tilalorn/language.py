@@ -193,7 +193,7 @@ class LanguageModel(RaggedLanguageModel):
                 if ns.moe:
                     z = self._linear(h2, ns.router, out_dtype=torch.float32)
                     route, _, _ = ops.moe_route_scored(z, ns.top, ns.groups, ns.keep, ns.rscale)
-                    if h2.numel() >= self.GROUPED_SIZE and ops.moe_grouped_fits(h2, ns.wff, ns.down, ns.ff):
+                    if h2.numel() >= self.GROUPED_SIZE and ops.moe_grouped_fits(h2, ns.wff, ns.down, ns.ff, ns.E):
                         rows, slots = ops.moe_grouped_rows(h2, ns.wff, ns.down, route, ns.top, ops.GLU_SILU, ff=ns.ff, out_dtype=torch.float32)
                         h = ops.add_slots_rms_(x, rows, slots, mult, w=nxt, w_offset=1.0, eps=eps)
                         keep += [z, route, h2, rows, slots]

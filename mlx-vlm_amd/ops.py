@@ -871,9 +871,9 @@ def moe_plan(gate, top, shared=0):
     return tok, tile_expert, ntiles, slots
 
 
-def moe_grouped_fits(h, wup, wdown, ff):
-    """whether the pair-by-pair form takes these rows and stacked expert weights"""
-    return (h.dtype == torch.bfloat16 and wup.dtype == torch.bfloat16 and h.shape[1] % 64 == 0 and ff % 64 == 0 and wdown.shape[0] % 8 == 0
+def moe_grouped_fits(h, wup, wdown, ff, E):
+    """whether the pair-by-pair form takes these rows and stacked weights of E experts (shared ones among them; its plan takes up to 256)"""
+    return (E <= 256 and h.dtype == torch.bfloat16 and wup.dtype == torch.bfloat16 and h.shape[1] % 64 == 0 and ff % 64 == 0 and wdown.shape[0] % 8 == 0
             and h.stride(0) % 8 == 0 and wup.stride(0) % 8 == 0 and wdown.stride(0) % 8 == 0
             and (h.data_ptr() | wup.data_ptr() | wdown.data_ptr()) % 16 == 0)
 
@@ -886,8 +886,8 @@ def moe_grouped_rows(h, wup, wdown, gate, top, act, limit=float("inf"), ff=None,
     N, ff = wdown.shape[0], int(ff or wdown.shape[1] // E)
     per = 1 if act == MOE_RELU2 else 2
     _dev(h, wup, wdown, gate)
-    if h.shape[0] != T or wup.shape[0] < E * per * ff or wup.shape[1] != h.shape[1] or wdown.shape[1] < E * ff or not moe_grouped_fits(h, wup, wdown, ff):
-        raise _lib.VlmHipError("moe_grouped_rows: bf16 rows and stacked expert weights with K and ff multiples of 64 expected")
+    if h.shape[0] != T or wup.shape[0] < E * per * ff or wup.shape[1] != h.shape[1] or wdown.shape[1] < E * ff or not moe_grouped_fits(h, wup, wdown, ff, E):
+        raise _lib.VlmHipError("moe_grouped_rows: bf16 rows and stacked weights of up to 256 experts with K and ff multiples of 64 expected")
     tok, tile_expert, ntiles, slots = moe_plan(gate, top, shared)
     tiles = tile_expert.numel()
     mid = torch.empty(tiles * MOE_TILE, ff, dtype=torch.bfloat16, device=h.device)

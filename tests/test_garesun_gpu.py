@@ -725,3 +725,24 @@ def test_experts_pair_by_pair_against_all_of_them(tmp_path, family, lens):
                 c[0]._seq.release()
         assert not torch.equal(got[0], got[1])                 # (two routes)
         assert H.rel_rms(got[0], got[1].double(), 0.9) < 2 * TOL["bfloat16"]
+
+
+@pytest.mark.parametrize("family,experts", [("garesun", 256), ("tilalorn", 272)])
+def test_more_experts_than_the_plan_takes(tmp_path, family, experts):
+    """a prompt above the size from which pairs are evaluated, with more experts (shared ones counted) than a plan holds: every expert for every token, as for a
+    shorter prompt"""
+    from tests import tilalorn_helpers as TH
+
+    if family == "garesun":
+        cfg = H.config([H.layer("retention", ff=64, shared_ff=64, experts=experts)], width=64)
+        W = H.weights(cfg)
+    else:
+        cfg = TH.config([TH.attention(mlp=TH.moe(experts=experts, groups=2, keep=1, ff=64))], width=64)
+        W = TH.weights(cfg)
+    lm = _load(tmp_path, cfg, W, "bfloat16")
+    lm = getattr(lm, "language_model", lm)
+    got = []
+    for size in (1, 1 << 30):
+        lm.GROUPED_SIZE = size
+        got.append(_whole(lm, _ids(40, cfg["vocab"], 3)))
+    assert torch.equal(*got)
