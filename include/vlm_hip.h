@@ -758,8 +758,7 @@ int vlm_relu2_rows(const void* in, long ldi, void* out, long ldo, int rows, int 
  * T is (a reader that goes on in fp32, e.g. a short convolution over the normed rows). */
 int vlm_scaled_add_rms(void* x, const void* y, long ldy, float mult, const void* y2, long ldy2, float mult2, const void* w, float w_offset,
                        void* h, long ldh, int h_f32, int rows, int D, float eps, int dtype, void* stream);
-/* x[t] += mult * (y[t] + the sum of the fp32 rows rows32[slots[t][k]], negative slots: none; y may be NULL); then, with w, h as above.  y, w: T; D % 4
- * == 0, rows of x and rows32 in aligned 16-byte pieces and of y, w and h in pieces of four elements */
+/* x[t] += mult * (y[t] + the sum of the fp32 rows rows32[slots[t][k]], negative slots: none; y may be NULL); then, with w, h as above.  y, w: T */
 int vlm_add_slots_rms(void* x, const void* y, long ldy, const void* rows32, long ldr, const void* slots, int nslots, float mult, const void* w,
                       float w_offset, void* h, long ldh, int rows, int D, float eps, int dtype, void* stream);
 

@@ -700,6 +700,22 @@ def test_pairs_with_a_shared_expert_and_fp32_rows(T, K, E, top, ff, N, shared, a
                 assert (hh.cpu().double() - nr).norm() < 2.0 ** -8 * nr.norm()
 
 
+@pytest.mark.parametrize("D", [16384, 16392, 70])
+def test_slots_step_of_any_width(D):
+    """rows wider than a workgroup's registers hold, and rows that do not come in pieces of four; three fp32 additions and the norm's rounding"""
+    from mlx_vlm_amd import ops
+
+    g = torch.Generator().manual_seed(D)
+    x, rows, y, w = (torch.randn(n, D, generator=g) for n in (3, 5, 3, 1))
+    y, w, slots = y.bfloat16().cuda(), w[0].bfloat16().cuda(), torch.tensor([[0, 4], [-1, 2], [-1, -1]], dtype=torch.int32)
+    got = x.clone().cuda()
+    h = ops.add_slots_rms_(got, rows.cuda(), slots.cuda(), 0.5, y=y, w=w, w_offset=1.0, eps=1e-6)
+    want = x.double() + 0.5 * (y.cpu().double() + torch.stack([sum((rows[s].double() for s in t if s >= 0), torch.zeros(D, dtype=F64)) for t in slots.tolist()]))
+    assert (got.cpu().double() - want).abs().max() <= 2.0 ** -21
+    nr = want / torch.sqrt(want.pow(2).mean(-1, keepdim=True) + 1e-6) * (1 + w.cpu().double())
+    assert ((h.cpu().double() - nr).abs() <= nr.abs() * 2.0 ** -8 + 1e-6).all()
+
+
 @pytest.mark.parametrize("family", ["garesun", "tilalorn"])
 @pytest.mark.parametrize("lens", [[64], [131, 5, 70], [300, 1]])
 def test_experts_pair_by_pair_against_all_of_them(tmp_path, family, lens):
