@@ -120,13 +120,19 @@ class LanguageModel(RaggedLanguageModel):
     def make_cache_batch(self, n: int):
         return [self.make_cache() for _ in range(n)]
 
-    def _workspace(self, pl, entries, per_token):
-        """room for the chunk-parallel recurrences of a step with prompt portions: `per_token` fp32 values a token and `entries` per chunk, the
-        latter up to 256 MB (longer prompts run in windows of chunks).  float32 serving stays token by token: the same bits however a prompt is cut"""
-        if pl.Tn - pl.nseg < 16:                              # decode rows and short portions only
+    def _workspace(self, pl):
+        """room for the chunk-parallel recurrences of a step with prompt portions, one piece for all layers (they follow each other on the stream): 2 H D fp32
+        values a token (rotated q and k) or 4 H (gates), and H D columns per chunk of 64 tokens, the latter up to 256 MB (longer prompts run in windows of
+        chunks).  float32 serving stays token by token: the same bits however a prompt is cut"""
+        layers = [ns for ns in self._L if ns.type in ("retention", "mlstm")]
+        if pl.Tn - pl.nseg < 16 or not layers or self.dtype == torch.float32:             # (decode rows and short portions only)
             return None
-        chunks = pl.Tn // 64 + pl.nseg
-        return torch.empty(per_token * pl.Tn + 4 + min(chunks, max(1, (64 << 20) // entries)) * entries, dtype=torch.float32, device=self.device)
+        chunks, need = pl.Tn // 64 + pl.nseg, 0
+        for ns in layers:
+            gated = ns.type == "mlstm"
+            entries, per_token = ns.H * ns.D * (ns.Dv + gated), 4 * ns.H if gated else 2 * ns.H * ns.D if ns.rot_dims else 0
+            need = max(need, per_token * pl.Tn + 4 + min(chunks, max(1, (64 << 20) // entries)) * entries)
+        return torch.empty(need, dtype=torch.float32, device=self.device)
 
     def _experts_grouped(self, ns, h):
         """whether a step's experts are evaluated pair by pair (the shared feed-forward as one more expert, which every token takes)"""
@@ -144,7 +150,8 @@ class LanguageModel(RaggedLanguageModel):
         is32 = T == f32
         few = Tn <= self.STREAM_ROWS and not is32           # decode rows over bf16 weights: weight-streaming projections with the expert skip
         x = ops.embed_scale_f32(ids_d, self._w["embed"], cfg.embedding_scale)
-        keep = [pl.md, ids_d]
+        ws = self._workspace(pl)
+        keep = [pl.md, ids_d, ws]
         for i, ns in enumerate(self._L):
             h = ops.layernorm_nobias(x, ns.norm1, cfg.norm_eps)
             gate = None
@@ -182,11 +189,10 @@ class LanguageModel(RaggedLanguageModel):
                 a.seg_start, a.seg_slot, a.seg_pos0 = cu_d.data_ptr(), slot_d.data_ptr(), pos0_d.data_ptr()
                 a.state, a.raw, a.out, a.ldo = pool.state[i].data_ptr(), raw.data_ptr(), cat.data_ptr(), cat.stride(0)
                 a.H, a.D, a.Dv, a.gated = ns.H, ns.D, ns.Dv, int(gated)
-                ws = None if is32 else self._workspace(pl, ns.H * ns.D * Cc, 4 * ns.H if gated else 2 * ns.H * ns.D if ns.rot_dims else 0)
                 if ws is not None:
                     a.ws, a.ws_floats = ws.data_ptr(), ws.numel()
                 ops.linear_recurrence(a, nseg, Tn, is32)
-                keep += [raw, ws]
+                keep.append(raw)
             else:
                 H, D, Dr, Dv, R = ns.H, ns.D, ns.Dr, ns.Dv, ns.R
                 if ns.src == i:

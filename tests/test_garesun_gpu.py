@@ -273,6 +273,18 @@ def test_a_workspace_changes_no_recurrence(gated, rot, q_act, decays):
         assert (got - want).abs().max() <= want.abs().max() * 2.0 ** -18
 
 
+def test_one_workspace_serves_all_recurrent_layers(tmp_path):
+    """a prompt over four recurrent layers of two kinds: what the step holds on to has one workspace, as large as the neediest layer's"""
+    cfg = H.config([H.layer("retention"), H.layer("mlstm"), H.layer("retention", heads=2, dim=40), H.layer("mlstm")])
+    lm = _load(tmp_path, cfg, H.weights(cfg), "bfloat16")
+    lm = getattr(lm, "language_model", lm)
+    T = 200
+    _whole(lm, _ids(T, cfg["vocab"], 1))
+    flat = [x.numel() for x in lm._keep if isinstance(x, torch.Tensor) and x.dtype == torch.float32 and x.dim() == 1]
+    need = [(4 * ns.H if ns.type == "mlstm" else 2 * ns.H * ns.D) * T + 4 + (T // 64 + 1) * ns.H * ns.D * (ns.Dv + (ns.type == "mlstm")) for ns in lm._L]
+    assert flat == [max(need)]
+
+
 # ------------------------------------------------------------------------------------------------ schedules
 @pytest.fixture(scope="module")
 def mixed32(tmp_path_factory):
