@@ -595,7 +595,8 @@ def gemm_rows(a, w, out=None):
     N = w.shape[0]
     if out is None:
         out = torch.empty(M, N, dtype=torch.bfloat16, device=a.device)
-    ws = torch.empty(8 * M * N if M <= 64 and K >= 1024 and N < 16384 else 0, dtype=torch.float32, device=a.device)
+    parts = 0 if M > 64 or K < 1024 else 8 if N < 16384 else 3 if N < 40960 and K >= 16384 else 0          # (the most that the split rule makes of these)
+    ws = torch.empty(parts * M * N, dtype=torch.float32, device=a.device)
     check(_lib.lib().vlm_gemm_bf16_ws(_p(a), _p(w), _p(out), M, N, K, a.stride(0), w.stride(0), out.stride(0), _p(ws), ws.numel() * 4, _stream()), "gemm")
     return out
 

@@ -674,6 +674,26 @@ def test_gemm_rows_splits_a_long_k_in_a_capture_too(M, N, K):
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("M,N,K", [(2, 16384, 16384), (64, 16448, 16384), (3, 16320, 16384), (2, 41024, 16384)])
+def test_gemm_rows_of_many_columns_in_a_capture(M, N, K):
+    """both sides of the lines in columns up to which a very long K is split: the captured product has the bits of the eager one"""
+    from mlx_vlm_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, w = (torch.randn(n, K, generator=g, device="cuda").bfloat16() for n in (M, N))
+    want, out = ops.gemm_rows(a, w), torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    ref = a.double() @ w[:512].double().T
+    assert (want[:, :512].double() - ref).norm() <= 2.0 ** -8 * ref.norm()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ops.gemm_rows(a, w, out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
 # ------------------------------------------------------------------------------------------------ experts of prompts, pair by pair
 @pytest.mark.parametrize("T,K,E,top,ff,N,shared", [(300, 128, 5, 2, 64, 72, 1), (70, 64, 3, 3, 128, 64, 0), (65, 192, 40, 4, 192, 264, 1), (513, 64, 0, 0, 64, 8, 1)])
 @pytest.mark.parametrize("act", [1, 5])
