@@ -43,22 +43,39 @@ __device__ __forceinline__ float elem(const u32x4_t& v, int e) {
   return e & 1 ? bf_hi(u) : bf_lo(u);
 }
 __device__ __forceinline__ f32x8_t join(f32x4_t lo, f32x4_t hi) { return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7); }
-__device__ __forceinline__ f32x4_t first4(f32x8_t v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3); }
+// (a vector type of an element's alignment: rows that are not whole aligned pieces are read in 16-byte accesses all the same)
+typedef f32x4_t f32x4_at4_t __attribute__((aligned(4)));
+typedef u32x4_t u32x4_at2_t __attribute__((aligned(2)));
 template <typename T, bool VEC>
 __device__ __forceinline__ Piece<T> piece(const T* p, int left) {          // left: elements before K
   if constexpr (VEC) {
     if constexpr (sizeof(T) == 4) return join(*reinterpret_cast<const f32x4_t*>(p), *reinterpret_cast<const f32x4_t*>(p + 4));
     else return *reinterpret_cast<const u32x4_t*>(p);
   } else if constexpr (sizeof(T) == 4) {
+    if (left >= 8) return join(*reinterpret_cast<const f32x4_at4_t*>(p), *reinterpret_cast<const f32x4_at4_t*>(p + 4));
     f32x8_t r;
 #pragma unroll
     for (int j = 0; j < 8; ++j) r[j] = j < left ? p[j] : 0.f;
     return r;
   } else {
+    if (left >= 8) return *reinterpret_cast<const u32x4_at2_t*>(p);
     u32x4_t r;
 #pragma unroll
     for (int j = 0; j < 4; ++j) r[j] = (2 * j < left ? (unsigned)p[2 * j] : 0u) | (2 * j + 1 < left ? (unsigned)p[2 * j + 1] << 16 : 0u);
     return r;
+  }
+}
+// the 16 bytes of a piece that begin at p (fp32: half of one)
+template <typename T>
+__device__ __forceinline__ u32x4_t bytes16(const T* p, int left) {
+  if constexpr (sizeof(T) == 4) {
+    if (left >= 4) return __builtin_bit_cast(u32x4_t, (f32x4_t)*reinterpret_cast<const f32x4_at4_t*>(p));
+    f32x4_t r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[j] = j < left ? p[j] : 0.f;
+    return __builtin_bit_cast(u32x4_t, r);
+  } else {
+    return piece<T, false>(p, left);
   }
 }
 __device__ __forceinline__ f32x4_t mfma_f32(float w, float a, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(w, a, c, 0, 0, 0); }
@@ -165,8 +182,9 @@ __global__ __launch_bounds__(64 * FW) void linear_f32_ranges_kernel(const TA* __
 
 // a workgroup: one tile of 2 MI x 2 NJ products on two groups of 2 x 2 waves, group q runs ranges 4 q .. 4 q + 3 over its own stages of LDS.
 // A slab arrives in LDS by 16-byte direct loads in the operand order (16 rows x 64 lanes per load), so that an operand is one linear read;
-// ST slabs are resident, ST - 2 in flight under the products.
-template <typename TA, typename TW, typename TC, int MI, int NJ, int ST>
+// ST slabs are resident, ST - 2 in flight under the products.  VEC: rows in whole aligned 16-byte pieces; others pass through registers, the next slab's
+// loads under this one's products (ST = 2).
+template <typename TA, typename TW, typename TC, int MI, int NJ, int ST, bool VEC>
 __global__ __launch_bounds__(512) void linear_f32_tiles_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N, int K,
                                                                long lda, long ldw, long ldc, long sA, long sW, long sC, int accumulate, int mtiles,
                                                                int ntiles) {
@@ -192,6 +210,19 @@ __global__ __launch_bounds__(512) void linear_f32_tiles_kernel(const TA* __restr
   }
   const int slabs = (K + FS - 1) / FS, range = (slabs + FW - 1) / FW;
   const int s0 = min(q * 4 * range, slabs), s1 = min(s0 + 4 * range, slabs), cnt = s1 - s0, steps = min(4 * range, slabs);
+  u32x4_t held[PER];
+  const auto fetch = [&](int s) {                                      // this wave's pieces of slab s to registers, zeros past K
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int t = min(wave + 4 * u, L - 1);
+      const int half = t < LA ? t % HA : (t - LA) % HW, left = K - s * FS - 8 * g - 4 * half;
+      held[u] = t < LA ? bytes16(reinterpret_cast<const TA*>(src[u]) + (size_t)s * FS, left) : bytes16(reinterpret_cast<const TW*>(src[u]) + (size_t)s * FS, left);
+    }
+  };
+  const auto put = [&](char* dst) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) *reinterpret_cast<u32x4_t*>(dst + min(wave + 4 * u, L - 1) * 1024 + lane * 16) = held[u];
+  };
   const auto issue = [&](int i) {                                      // slab s0 + i
     const int s = s0 + i;
     char* dst = base + (size_t)(i % ST) * L * 1024;
@@ -202,23 +233,9 @@ __global__ __launch_bounds__(512) void linear_f32_tiles_kernel(const TA* __restr
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[u] + (size_t)s * FS * (t < LA ? sizeof(TA) : sizeof(TW))),
                                          (__attribute__((address_space(3))) void*)(dst + t * 1024), 16, 0, 0);
       }
-    } else {                                                           // the last, shorter slab: zeros past K
-#pragma unroll
-      for (int u = 0; u < PER; ++u) {
-        const int t = min(wave + 4 * u, L - 1);
-        const int half = t < LA ? t % HA : (t - LA) % HW, left = K - s * FS - 8 * g - 4 * half;
-        u32x4_t v;
-        if (t < LA) {
-          const TA* p = reinterpret_cast<const TA*>(src[u]) + (size_t)s * FS;
-          const Piece<TA> r = piece<TA, false>(p, sizeof(TA) == 4 ? min(left, 4) : left);
-          if constexpr (sizeof(TA) == 4) v = __builtin_bit_cast(u32x4_t, first4(r)); else v = r;
-        } else {
-          const TW* p = reinterpret_cast<const TW*>(src[u]) + (size_t)s * FS;
-          const Piece<TW> r = piece<TW, false>(p, sizeof(TW) == 4 ? min(left, 4) : left);
-          if constexpr (sizeof(TW) == 4) v = __builtin_bit_cast(u32x4_t, first4(r)); else v = r;
-        }
-        *reinterpret_cast<u32x4_t*>(dst + t * 1024 + lane * 16) = v;
-      }
+    } else {                                                           // the last, shorter slab
+      fetch(s);
+      put(dst);
     }
   };
   f32x4_t acc[MI][NJ], tot[MI][NJ];
@@ -226,15 +243,24 @@ __global__ __launch_bounds__(512) void linear_f32_tiles_kernel(const TA* __restr
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = tot[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if constexpr (VEC) {
 #pragma unroll
-  for (int i = 0; i < ST - 1; ++i)
-    if (i < cnt) issue(i);
+    for (int i = 0; i < ST - 1; ++i)
+      if (i < cnt) issue(i);
+  } else if (cnt > 0) {
+    fetch(s0);
+    put(base);
+  }
   int in_range = 0;
   for (int i = 0; i < steps; ++i) {
-    if (i + ST - 2 < cnt) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((ST - 2) * PER) : "memory");
+    if (VEC && i + ST - 2 < cnt) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((ST - 2) * PER) : "memory");
     else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();                                      // slab i is there for every wave, and everybody is done with slab i - 1
-    if (i + ST - 1 < cnt) issue(i + ST - 1);
+    if constexpr (VEC) {
+      if (i + ST - 1 < cnt) issue(i + ST - 1);
+    } else {
+      if (i + 1 < cnt) fetch(s0 + i + 1);                              // (in flight under the products)
+    }
     if (i < cnt) {
       const char* st = base + (size_t)(i % ST) * L * 1024 + lane * 16;
       Piece<TA> a[MI];
@@ -268,6 +294,7 @@ __global__ __launch_bounds__(512) void linear_f32_tiles_kernel(const TA* __restr
           }
       }
     }
+    if (!VEC && i + 1 < cnt) put(base + (size_t)((i + 1) % ST) * L * 1024);
   }
   // the second group's sums through LDS (the stages' place)
   __syncthreads();
@@ -314,12 +341,13 @@ int launch_f32(const void* A, const void* W, void* C, int M, int N, int K, long 
                        sC, accumulate, (int)mt, (int)nt);                                                                           \
   } while (0)
 #define RANGES(MI, NJ, VEC) GO((linear_f32_ranges_kernel<TA, TW, TC, MI, NJ, VEC>), 16 * MI, 16 * NJ, 0)
-#define TILES(MI, NJ, ST)                                                                                                           \
+#define TILES(MI, NJ, ST, VEC)                                                                                                      \
   do {                                                                                                                              \
-    constexpr int lds = 2 * ST * (2 * MI * (int)sizeof(TA) / 2 + 2 * NJ * (int)sizeof(TW) / 2) * 1024;                              \
-    const hipError_t e = hipFuncSetAttribute((const void*)linear_f32_tiles_kernel<TA, TW, TC, MI, NJ, ST>, hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+    constexpr int stages = VEC ? ST : 2, lds = 2 * stages * (2 * MI * (int)sizeof(TA) / 2 + 2 * NJ * (int)sizeof(TW) / 2) * 1024;   \
+    const hipError_t e = hipFuncSetAttribute((const void*)linear_f32_tiles_kernel<TA, TW, TC, MI, NJ, stages, VEC>,                 \
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);                                      \
     if (e != hipSuccess) return VLM_ERR_HIP + (int)e;                                                                               \
-    GO((linear_f32_tiles_kernel<TA, TW, TC, MI, NJ, ST>), 32 * MI, 32 * NJ, lds);                                                   \
+    GO((linear_f32_tiles_kernel<TA, TW, TC, MI, NJ, stages, VEC>), 32 * MI, 32 * NJ, lds);                                          \
   } while (0)
   // Where the lines lie (us of one call; the kernel of scalar FMAs that stood here | ranges 16 x 16 | tiles 32 x 64 | 64 x 64 | 64 x 128):
   //   301 rows, W [26304, 1536] fp32            881 | 1272 | 410 | 357 | 351        1 row, the same W              185 |  51 |  48 |  74 |  69
@@ -327,13 +355,18 @@ int launch_f32(const void* A, const void* W, void* C, int M, int N, int K, long 
   //   400 rows, W [41000, 3584] fp32           3987 | 3910 | 1626 | 1488 | 1335     2048 rows, W [1536, 1536]      333 | 510 | 149 | 123 | 142
   //   301 rows, 12 maps [512, 128] fp32          25 |   89 |  17 |  13 |  20        2048 rows, 12 maps [128, 512] bf16  110 | 191 | 43 | 39 | 50
   //   2048 rows, W [64, 1536] bf16               95 |   19 |  23 |  37 |  64  (ranges 32 x 32: 14)
-  // a wide tile reads its operands less often, a narrow one leaves fewer compute units without work
-  if (!vec) RANGES(2, 2, false);
-  else if (M > 32 && tiles(64, 128) >= 768) TILES(2, 4, 3);
-  else if (M > 32 && tiles(64, 64) >= 448) TILES(2, 2, 3);
-  else if (tiles(32, 64) >= 160) TILES(1, 2, 4);
-  else if (M > 16 && tiles(32, 32) >= 128) RANGES(2, 2, true);
-  else RANGES(1, 1, true);
+  // a wide tile reads its operands less often, a narrow one leaves fewer compute units without work.
+  // Rows that are not whole aligned pieces come through registers (scalar FMAs | ranges 32 x 32, as all of them ran | tiles 32 x 64 | 64 x 64 | 64 x 128):
+  //   301 rows, W [1536, 1537] fp32            119 |  40 |  29 |  44 |  75          2048 rows, W [6144, 1539] bf16     757 | 863 | 690 | 398 | 444
+  //   301 rows, W [26304, 1537] fp32           849 | 570 | 335 | 311 | 348          2048 rows, 12 maps [512, 129]      109 | 242 |  76 |  65 |  71
+  //   1 row, W [1536, 21699] fp32             2027 | 152 | 299 | 457 | 845  (ranges 16 x 16: 50)
+#define BY(KIND, ...) do { if (vec) KIND(__VA_ARGS__, true); else KIND(__VA_ARGS__, false); } while (0)
+  if (vec && M > 32 && tiles(64, 128) >= 768) TILES(2, 4, 3, true);
+  else if (M > 32 && tiles(64, 64) >= 448) BY(TILES, 2, 2, 3);
+  else if (tiles(32, 64) >= 160) BY(TILES, 1, 2, 4);
+  else if (M > 16 && tiles(32, 32) >= 128) BY(RANGES, 2, 2);
+  else BY(RANGES, 1, 1);
+#undef BY
 #undef TILES
 #undef RANGES
 #undef GO

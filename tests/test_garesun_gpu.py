@@ -94,6 +94,35 @@ def test_linear_any_f32_tiles(M, N, K):
     assert torch.equal(ops.linear_any(b, w), ops.linear_any(b.contiguous(), w) if K % 4 == 0 else ops.linear_any(b.clone(), w))
 
 
+@pytest.mark.parametrize("M, N, K, batch", [(1, 40, 33, 1), (17, 260, 40, 1), (33, 1030, 97, 1), (100, 7000, 37, 1), (300, 600, 1031, 1), (70, 520, 129, 12), (257, 64, 515, 3), (65, 4100, 8, 1)])
+@pytest.mark.parametrize("ta,tw", [("float32", "float32"), ("float32", "bfloat16"), ("bfloat16", "float32"), ("bfloat16", "bfloat16")])
+def test_rows_that_are_not_whole_pieces_have_the_bits_of_those_that_are(M, N, K, batch, ta, tw):
+    """every tile shape over rows at odd pitches and odd addresses, against the same rows padded to whole 16-byte pieces (zeros past K: the same chains).  (bf16 times
+    bf16 rows take other kernels when they are aligned: against float64 there)"""
+    from mlx_vlm_amd import ops
+
+    g = torch.Generator().manual_seed(M + N + K)
+    ta, tw = getattr(torch, ta), getattr(torch, tw)
+    a, w = torch.randn(M, batch, K, generator=g).to(ta), torch.randn(batch, N, K, generator=g).to(tw)
+    K8 = (K + 7) & ~7
+    out, got = [], None
+    for odd in (True, False):
+        pad = K + 1 - K % 2 if odd else K8                   # (an odd number)
+        abuf, wbuf = torch.zeros(M * batch * pad + 1, dtype=ta), torch.zeros(batch * N * pad + 1, dtype=tw)
+        av, wv = (b[int(odd):][: b.numel() - 1].view(-1, pad) for b in (abuf, wbuf))
+        av[:, :K], wv[:, :K] = a.reshape(-1, K), w.reshape(-1, K)
+        ad, wd = abuf.cuda()[int(odd):][: M * batch * pad].view(M, batch * pad), wbuf.cuda()[int(odd):][: batch * N * pad].view(batch * N, pad)
+        o = torch.empty(M, batch * N, device="cuda")
+        ops.linear_any(ad, wd, out=o, M=M, N=N, K=K, batch=batch, stride_a=pad, stride_w=N * pad, stride_c=N)
+        out.append(o)
+    if M > 1 and tw == torch.bfloat16:
+        ref = (a.double().transpose(0, 1) @ w.double().transpose(1, 2)).transpose(0, 1).reshape(M, batch * N).cuda()
+        room = (a.double().abs().transpose(0, 1) @ w.double().abs().transpose(1, 2)).transpose(0, 1).reshape(M, batch * N).cuda() * (K * 2.0 ** -24)
+        assert ((out[0].double() - ref).abs() <= room).all()
+    elif not (M <= 8 and (ta, tw) != (torch.float32, torch.float32)):
+        assert torch.equal(*out)
+
+
 def test_stream_row_operators():
     from mlx_vlm_amd import ops
 
