@@ -19,7 +19,7 @@
 // Scan work split: a state column's rows lie in the registers of 8 / 16 / 32 neighbouring lanes, workgroup = (segment, head, tile of columns) of four
 // waves; heads up to 1024 wide.  What bounds a long segment is the chain of one token - a dot product with the state, its sum over the lanes, the
 // update - times the tokens, so the rows are spread thin (768 waves for 12 heads of 128, where 16 rows a lane on 8 lanes, one sum after the other
-// and tokens staged behind a barrier took 1159 us for 1500 tokens in the general form and 831 us in the gated one: now 270 and 246), the sum of a
+// and tokens staged behind a barrier took 1159 us for 1500 tokens in the general form and 831 us in the gated one: now 265 and 240), the sum of a
 // read-out runs beside the next token's, and the tokens' vectors arrive in LDS by direct loads two blocks ahead.
 #include "common.hpp"
 #include "../../include/vlm_hip.h"
@@ -188,8 +188,10 @@ __device__ __forceinline__ void direct_load4(const float* src, float* dst) {
 }
 
 // lane = (column group lane / RG of the wave's 64 / RG, row group rg = lane % RG): rows [DR rg, DR rg + DR) of NC neighbouring state columns in
-// registers.  A token's vectors in LDS: [vector][token of the block][RG * DR], a lane reads its own rows.  VEC: D == RG * DR, the vectors' rows in
-// whole aligned 16-byte pieces, and state rows in pieces of NC; else both element by element, zeros past D.
+// registers.  A token's vectors in LDS: [vector][token of the block][RG * DR], a lane reads its own rows, four at a time; a lane's fours lie RG fours apart, so that
+// neighbouring lanes read neighbouring 16 bytes (as the rows come, lanes of 8 to 32 rows met in the same banks: general form, 4 x 30 tokens of 2 heads of 1024,
+// 96 us instead of 42).  WHOLE: D == RG * DR, the vectors' rows in whole aligned 16-byte pieces, and state rows in pieces of NC; FOURS: such vectors alone
+// (general form, D = 100, 700 + 700 tokens of 12 heads: 163 us, element by element 358); ANY: element by element.  Zeros past D.
 template <int DR, int RG, int NC, bool GENERAL> struct ScanShape {
   static constexpr int DP = RG * DR, NV = GENERAL ? 5 : 2;
   static constexpr int TB = DP > 128 ? 1024 / DP : NC == 1 || DP <= 32 ? 8 : 4, NBUF = 3;                // tokens per block, blocks resident
@@ -198,7 +200,8 @@ template <int DR, int RG, int NC, bool GENERAL> struct ScanShape {
   static_assert(TB * DP % 256 == 0, "a direct load is 256 floats of one vector");
 };
 
-template <int DR, int RG, int NC, bool GENERAL, bool VEC>
+enum { ANY, FOURS, WHOLE };
+template <int DR, int RG, int NC, bool GENERAL, int MODE>
 __global__ __launch_bounds__(256) void delta_scan_kernel(vlm_delta_rule_args p) {
   extern __shared__ __align__(16) float smem[];
   using SS = ScanShape<DR, RG, NC, GENERAL>;
@@ -215,7 +218,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(vlm_delta_rule_args p) 
   const auto vec = [&](int n) { return n == 0 ? p.kw : n == 1 || !GENERAL ? p.q : n == 2 ? p.kr : n == 3 ? p.w : p.b; };
   float* S = p.state + ((long)slot * p.H + h) * (long)D * Dv;
   float s[NC][DR];
-  if constexpr (VEC) {
+  if constexpr (MODE == WHOLE) {
     typedef float pc_t __attribute__((ext_vector_type(NC)));
 #pragma unroll
     for (int r = 0; r < DR; ++r) {
@@ -230,28 +233,29 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(vlm_delta_rule_args p) 
 #pragma unroll
       for (int c = 0; c < NC; ++c) s[c][r] = (pos0 > 0 && row0 + r < D && col + c < Dv) ? S[(long)(row0 + r) * Dv + col + c] : 0.f;
   }
+  const auto row_of = [](int e) { return (e / 4 % RG * (DR / 4) + e / 4 / RG) * 4 + e % 4; };          // of element e of a vector in LDS
   const float* src[PER];                                             // where this lane's direct loads start
-  if constexpr (VEC)
+  if constexpr (MODE != ANY)
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
       const int l = min(wave + 4 * u, SS::LOADS - 1);
-      src[u] = vec(l / (TB * DP / 256)) + (long)kh * D + lane * 4 % DP;
+      src[u] = vec(l / (TB * DP / 256)) + (long)kh * D + row_of((l * 256 + lane * 4) % DP);
     }
   const float* vsrc = p.v + (long)h * Dv;
   const float* gsrc = GENERAL ? nullptr : (lane & 1 ? p.beta : p.g) + h;
   const auto issue = [&](int i) {                                    // block i into its buffer (tokens past the end: the last one again)
     float* buf = smem + (i % NBUF) * BLOCK;
     const int t0 = t_begin + i * TB;
-    if constexpr (VEC) {
+    if constexpr (MODE != ANY) {
 #pragma unroll
-      for (int u = 0; u < PER; ++u) {
-        const int l = min(wave + 4 * u, SS::LOADS - 1), t = (l * 256 + lane * 4) / DP % TB;
-        direct_load16(src[u] + (long)min(t0 + t, t_end - 1) * p.ldk + (DP > 256 ? l * 256 % DP : 0), buf + l * 256);
+      for (int u = 0; u < PER; ++u) {                                // (every load has a row below D, its first: none is left out by a wave)
+        const int l = min(wave + 4 * u, SS::LOADS - 1), e = l * 256 + lane * 4, t = e / DP % TB;
+        if (MODE == WHOLE || row_of(e % DP) < D) direct_load16(src[u] + (long)min(t0 + t, t_end - 1) * p.ldk, buf + l * 256);
       }
     } else {
 #pragma unroll 4
       for (int base = wave * 64; base < VECS; base += 256) {
-        const int f = base + lane, t = f / DP % TB, row = f % DP;
+        const int f = base + lane, t = f / DP % TB, row = row_of(f % DP);
         if (row < D) direct_load4(vec(base / (TB * DP)) + (long)min(t0 + t, t_end - 1) * p.ldk + (long)kh * D + row, buf + base);
       }
     }
@@ -263,14 +267,12 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(vlm_delta_rule_args p) 
     if constexpr (!GENERAL)
       if (lane < 2 * TB) direct_load4(gsrc + (long)min(t0 + lane / 2, t_end - 1) * p.H, buf + VECS + TB * CT);
   };
-  if constexpr (VEC) {
-    if (blocks > 1) issue(0), issue(1);
-    else if (blocks > 0) issue(0);
-  } else {
+  if constexpr (MODE != WHOLE) {
     for (int f = tid; f < NBUF * BLOCK; f += 256) smem[f] = 0.f;     // (rows past D stay zero)
     __syncthreads();
-    if (blocks > 0) issue(0);
   }
+  if (blocks > 0) issue(0);
+  if (MODE != ANY && blocks > 1) issue(1);
   // (the state has to be waited for here: inside the loop that wait would be for the direct loads too)
 #pragma unroll
   for (int r = 0; r < DR; ++r)
@@ -278,7 +280,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(vlm_delta_rule_args p) 
     for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(s[c][r]));
   struct Token { f32x4_t k[DR / 4], q[DR / 4], u[DR / 4], w[DR / 4], b[DR / 4]; float v[NC], g, beta; };
   for (int i = 0; i < blocks; ++i) {
-    if constexpr (VEC) {
+    if constexpr (MODE != ANY) {
       // (stores of read-outs may be among what is waited for; direct loads return in order)
       if (i + 1 < blocks) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(ISSUED) : "memory");
       else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
@@ -294,17 +296,17 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(vlm_delta_rule_args p) 
     float mine[NC] = {};                                             // the read-outs of token rg of the block
     const auto load = [&](int t) {
       Token x;
-      const f32x4_t* row = reinterpret_cast<const f32x4_t*>(buf + t * DP + row0);
+      const f32x4_t* row = reinterpret_cast<const f32x4_t*>(buf + t * DP) + rg;
       constexpr int V = TB * DP / 4;
 #pragma unroll
       for (int r = 0; r < DR / 4; ++r) {
         if constexpr (GENERAL) {
-          x.u[r] = row[r + 2 * V];
-          x.w[r] = row[r + 3 * V];
-          x.b[r] = row[r + 4 * V];
+          x.u[r] = row[RG * r + 2 * V];
+          x.w[r] = row[RG * r + 3 * V];
+          x.b[r] = row[RG * r + 4 * V];
         }
-        x.k[r] = row[r];
-        x.q[r] = row[r + V];
+        x.k[r] = row[RG * r];
+        x.q[r] = row[RG * r + V];
       }
       if constexpr (!GENERAL) {
         x.g = buf[VECS + TB * CT + 2 * t];
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(vlm_delta_rule_args p) 
   }
 #pragma unroll
   for (int r = 0; r < DR; ++r) {
-    if constexpr (VEC) {
+    if constexpr (MODE == WHOLE) {
       typedef float pc_t __attribute__((ext_vector_type(NC)));
       pc_t x;
 #pragma unroll
@@ -390,35 +392,54 @@ int launch_scan(const vlm_delta_rule_args& a, int nseg, hipStream_t st) {
   constexpr int CT = 256 / RG * NC;
   constexpr size_t lds = (size_t)SS::NBUF * SS::BLOCK * sizeof(float);
   const uintptr_t ptrs = (uintptr_t)a.kw | (uintptr_t)a.q | (uintptr_t)a.state | (GENERAL ? (uintptr_t)a.kr | (uintptr_t)a.w | (uintptr_t)a.b : 0);
-  const bool vec = a.D == SS::DP && a.ldk % 4 == 0 && a.Dv % NC == 0 && ptrs % 16 == 0;
+  const bool fours = a.D % 4 == 0 && a.ldk % 4 == 0 && ptrs % 16 == 0;           // the vectors' rows in whole aligned 16-byte pieces
+  const bool whole = fours && a.D == SS::DP && a.Dv % NC == 0;
   const dim3 grid(nseg, a.H, (a.Dv + CT - 1) / CT), block(256);
   static_assert(lds <= 64 * 1024, "");
-  if (vec) hipLaunchKernelGGL((delta_scan_kernel<DR, RG, NC, GENERAL, true>), grid, block, lds, st, a);
-  else hipLaunchKernelGGL((delta_scan_kernel<DR, RG, NC, GENERAL, false>), grid, block, lds, st, a);
+  if (whole) hipLaunchKernelGGL((delta_scan_kernel<DR, RG, NC, GENERAL, WHOLE>), grid, block, lds, st, a);
+  else if (fours) hipLaunchKernelGGL((delta_scan_kernel<DR, RG, NC, GENERAL, FOURS>), grid, block, lds, st, a);
+  else hipLaunchKernelGGL((delta_scan_kernel<DR, RG, NC, GENERAL, ANY>), grid, block, lds, st, a);
   VLM_CHECK_LAUNCH();
   return VLM_OK;
 }
 
-// Which spread of the state, for heads of 128 (rows a lane, lanes a column, columns a lane; the results are the same bits in all of them).  (4, 32, 1)
-// keeps a token's chain shortest: 1500 tokens of 12 heads 270 us (general) and 246 us (gated), against 354 and 286 with (8, 16, 1), 409 and 380 with
-// (4, 32, 2).  Segments of a few tokens move more state than they compute and take pieces of 32 bytes of a state row a wave: 32 sequences of one
-// token, 28 heads: (4, 32, 4) 30 us, (4, 32, 1) 85.  With more workgroups than are resident at once the work counts, not the chain: the general form
-// reads five vectors a token from LDS and shares them between columns (1100 + 333 + 70 tokens of 28 heads: (4, 32, 2) 379 us, (4, 32, 1) 450), the gated
-// one saves on sums over lanes ((8, 16, 1) 264 us, (4, 32, 1) 302); many times as many: 32 sequences of 20 tokens, 28 heads, gated:
-// (16, 8, 1) 79 us, (8, 16, 1) 97, (4, 32, 1) 119.
+// Which spread of the state (rows a lane, lanes a column, columns a lane; the results are the same bits in all of them).  Heads of 128: (4, 32, 1) keeps a token's
+// chain shortest: 1500 tokens of 12 heads 265 us (general) and 240 us (gated), against 354 and 286 with (8, 16, 1), 409 and 380 with (4, 32, 2).  Segments of a few
+// tokens move more state than they compute and take pieces of 32 bytes of a state row a wave: 32 sequences of one token, 28 heads: (4, 32, 4) 30 us,
+// (4, 32, 1) 85.  With more workgroups than are resident at once the work counts, not the chain: fewer lanes save on sums over them, and the general form reads
+// five vectors a token from LDS and shares them between columns.  us, sequences x tokens x heads (`groups`); "before": 16 rows a lane on 8 lanes, tokens behind a barrier:
+//   gated 128    3 (1100 + 333 + 70) x 28 (1344)  before 625  (8, 16, 1) 232  (16, 8, 1) 310    4 x 200 x 28 (1792)   132   91   85     16 x 100 x 28 (7168)  153  153  136
+//                32 x 40 x 12 (6144)                      59              60              54    16 x 60 x 12 (3072)    53   50   44     32 x 20 x 28 (14336)   76   75   75
+//   general 128  3 (1100 + 333 + 70) x 28         before 868  (4, 32, 2) 355  (8, 16, 2) 445    4 x 200 x 28          174  141  126     16 x 100 x 28         221  234  186
+//                32 x 40 x 12                             92              85              73    16 x 60 x 12           67   68   59     32 x 20 x 28          103  106   86
+//   gated 64     3 (1100 + 333 + 70) x 28 (672)   before 452  (4, 16, 1) 155  (8, 8, 1) 189     8 x 300 x 28 (1792)   140   96   84     32 x 20 x 28 (7168)    32   35   28
+//   gated 256    3 (1100 + 333 + 70) x 14 (1344)  before 1007 (8, 32, 1) 407  (16, 16, 1) 408   8 x 300 x 14 (3584)   387  454  362     16 x 100 x 14 (7168)  254  327  265
+//                                                             (16, 16, 2) 572                                              424                                        248
+//   general 256  3 (1100 + 333 + 70) x 14         before 1483 (8, 32, 2) 667  (16, 16, 2) 735   8 x 300 x 14          930  607  587     32 x 40 x 6 (6144)    148  159  134
+// (A step whose sequences differ much in length waits for the longest one's chain, which the shapes for many workgroups lengthen: the host knows only how many
+// tokens there are.)
 template <bool GENERAL>
 int run_scan(const vlm_delta_rule_args& a, int nseg, int ntok, hipStream_t st) {
   const bool few = ntok <= 16L * nseg;
+  const long groups = (long)nseg * a.H * ((a.Dv + 7) / 8);           // workgroups of eight columns
   if (a.D <= 32) return launch_scan<4, 8, 1, GENERAL>(a, nseg, st);
-  if (a.D <= 64) return few ? launch_scan<4, 16, 2, GENERAL>(a, nseg, st) : launch_scan<4, 16, 1, GENERAL>(a, nseg, st);
-  if (a.D <= 128) {
-    const long groups = (long)nseg * a.H * ((a.Dv + 7) / 8);         // workgroups of (4, 32, 1)
-    if (few) return launch_scan<4, 32, 4, GENERAL>(a, nseg, st);
-    if (groups > 8192) return launch_scan<16, 8, 1, GENERAL>(a, nseg, st);
-    if (groups > 1024) return GENERAL ? launch_scan<4, 32, 2, GENERAL>(a, nseg, st) : launch_scan<8, 16, 1, GENERAL>(a, nseg, st);
-    return launch_scan<4, 32, 1, GENERAL>(a, nseg, st);
+  if (a.D <= 64) {
+    if (few) return launch_scan<4, 16, 2, GENERAL>(a, nseg, st);
+    return groups > 2048 ? launch_scan<8, 8, 1, GENERAL>(a, nseg, st) : launch_scan<4, 16, 1, GENERAL>(a, nseg, st);
   }
-  if (a.D <= 256) return few ? launch_scan<8, 32, 4, GENERAL>(a, nseg, st) : launch_scan<8, 32, 1, GENERAL>(a, nseg, st);
+  if (a.D <= 128) {
+    if (few) return launch_scan<4, 32, 4, GENERAL>(a, nseg, st);
+    if (groups <= 1024) return launch_scan<4, 32, 1, GENERAL>(a, nseg, st);
+    if constexpr (GENERAL) return groups > 2048 ? launch_scan<8, 16, 2, true>(a, nseg, st) : launch_scan<4, 32, 2, true>(a, nseg, st);
+    else return groups > 4096 ? launch_scan<16, 8, 1, false>(a, nseg, st) : launch_scan<8, 16, 1, false>(a, nseg, st);
+  }
+  if (a.D <= 256) {
+    if (few) return launch_scan<8, 32, 4, GENERAL>(a, nseg, st);
+    if (groups <= (GENERAL ? 512 : 1024)) return launch_scan<8, 32, 1, GENERAL>(a, nseg, st);
+    if (groups > (GENERAL ? 2048 : 4096)) return launch_scan<16, 16, 2, GENERAL>(a, nseg, st);
+    if constexpr (GENERAL) return launch_scan<8, 32, 2, true>(a, nseg, st);
+    else return launch_scan<16, 16, 1, false>(a, nseg, st);
+  }
   if (a.D <= 512) return few ? launch_scan<16, 32, 2, GENERAL>(a, nseg, st) : launch_scan<16, 32, 1, GENERAL>(a, nseg, st);
   if (a.D <= 1024) return few ? launch_scan<32, 32, 2, GENERAL>(a, nseg, st) : launch_scan<32, 32, 1, GENERAL>(a, nseg, st);
   return VLM_ERR_SHAPE;

@@ -112,7 +112,10 @@ def test_stream_operators_at_the_widths_of_their_forms(T, D):
 
 @pytest.mark.parametrize("mode", [0, 1])
 @pytest.mark.parametrize("Hh,KH,D,Dv,many", [(3, 3, 20, 24, 1), (2, 2, 32, 33, 1), (4, 2, 64, 66, 1), (6, 3, 128, 130, 1), (12, 4, 128, 128, 1), (28, 28, 128, 128, 3),
-                                            (28, 14, 128, 64, 40), (3, 1, 100, 8, 1), (2, 2, 256, 20, 1), (2, 1, 300, 8, 1), (1, 1, 512, 9, 1), (1, 1, 1024, 8, 1)])
+                                            (28, 14, 128, 64, 40), (3, 1, 100, 8, 1), (2, 2, 256, 20, 1), (2, 1, 300, 8, 1), (1, 1, 512, 9, 1), (1, 1, 1024, 8, 1),
+                                            (28, 28, 64, 64, 5), (28, 28, 128, 128, 2), (28, 28, 128, 128, 5), (8, 8, 256, 128, 3), (8, 8, 256, 128, 5), (8, 8, 256, 128, 17),
+                                            (28, 14, 60, 64, 5), (28, 28, 100, 130, 5), (8, 4, 200, 132, 5), (8, 8, 200, 132, 17),
+                                            (2, 2, 50, 10, 1), (28, 28, 61, 64, 5), (28, 28, 99, 128, 2), (28, 28, 99, 128, 5), (8, 8, 201, 130, 17), (1, 1, 514, 9, 1)])
 def test_delta_rule_spreads_of_the_state(mode, Hh, KH, D, Dv, many):
     """segments of no, one and some tokens around the blocks of 4 and 8, fresh and carried states, alone (few tokens: one spread over the lanes),
     together (another) and `many` times over (others): the same bits, and within 2^-21 (rms) of float64 - sums of D products as a tree of fours are
