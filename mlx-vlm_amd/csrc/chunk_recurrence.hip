@@ -148,6 +148,7 @@ __global__ __launch_bounds__(256) void chunk_update_kernel(vlm_recurrence_args p
   }
   // tile (a, b): row 4 (4 g + r) + a, column 4 r16 + b of the super tile
   float* U = ws + ((long)blockIdx.x * p.H + h) * (long)D * (Dv + GATED);
+  const bool uvec = Dv % 4 == 0 && (((uintptr_t)U) & 15) == 0;          // (with a normaliser column a chunk's piece may begin anywhere)
   if constexpr (GATED) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(256) void chunk_update_kernel(vlm_recurrence_args p
       const int d = (st / sc) * 64 + 4 * (4 * g + r) + a;
       if (d >= D) continue;
       float* u = U + (long)d * Dv + v0;
-      if (Dv % 4 == 0) {
+      if (uvec) {
         if (v0 < Dv) *reinterpret_cast<float4*>(u) = make_float4(acc[a][0][r], acc[a][1][r], acc[a][2][r], acc[a][3][r]);
       } else {
 #pragma unroll

@@ -189,7 +189,7 @@ def test_layers_match_layer_by_layer(tmp_path, dtype):
         lm._trace = None
 
 
-@pytest.mark.parametrize("gated,rot,D,Dv,Hh", [(1, 0, 128, 128, 3), (1, 0, 40, 130, 2), (1, 0, 13, 7, 1), (0, 32, 32, 48, 3), (0, 20, 70, 16, 2), (0, 128, 128, 128, 2)])
+@pytest.mark.parametrize("gated,rot,D,Dv,Hh", [(1, 0, 128, 128, 3), (1, 0, 40, 130, 2), (1, 0, 13, 7, 1), (1, 0, 13, 8, 3), (0, 32, 32, 48, 3), (0, 20, 70, 16, 2), (0, 128, 128, 128, 2)])
 def test_chunk_parallel_recurrences_against_the_token_by_token_kernel(gated, rot, D, Dv, Hh):
     """segments around the borders of a chunk next to short ones, fresh and carried states, workspaces of one chunk and of all: read-outs, states
     and maxima against float64, no further off than 1.5 times the token-by-token kernel (or 2^-20 of the largest value: sums of another order)"""
