@@ -330,6 +330,11 @@ __global__ __launch_bounds__(256) void chunk_output_kernel(vlm_recurrence_args p
       for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(p.v_act ? silu_f(v[b]) : v[b], pr, acc[b], 0, 0, 0);
     }
   }
+  float odd = 0.f;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) odd = fmaf(acc[b][x], 0.f, odd);
   if constexpr (GATED) nq = fmaf(col4_sum(nq), ai, col4_sum(mine));
   if (i >= n) return;
   // block b, register r of lane group g: column (4 g + r) NB + b of the tile
@@ -347,6 +352,31 @@ __global__ __launch_bounds__(256) void chunk_output_kernel(vlm_recurrence_args p
       for (int b = 0; b < NB; ++b)
         if (c + b < Dv) o[c + b] = acc[b][r];
     }
+  }
+  if (!__any(odd != 0.f)) return;
+  // a value that is not finite met the zero weights of the queries before it in the last tile: these tokens' read-outs once more, without such products
+  const int first = blockIdx.z * 16 * NB + 4 * g * NB, last = min(first + 4 * NB, Dv);
+  const auto value = [](const auto* x, int act, float scale) {
+    float f;
+    row_vals<1>(x, 1, false, &f);
+    return (act ? silu_f(f) : f) * scale;
+  };
+#pragma unroll 1
+  for (int c = first; c < last; ++c) {
+    float x = 0.f;
+#pragma unroll 1
+    for (int d = 0; d < D; ++d) x = fmaf(S0[(long)d * Dv + c], value(qp + d, p.q_act, p.qscale), x);
+    o[c] = x * ai;
+  }
+#pragma unroll 1
+  for (int j = 0; j <= i; ++j) {
+    float x = 0.f;
+#pragma unroll 1
+    for (int d = 0; d < D; ++d) x = fmaf(value(kp + (long)j * p.ldk + d, p.k_act, p.kscale), value(qp + d, p.q_act, p.qscale), x);
+    const long tj = (long)(t0 + j) * p.H + h;
+    x *= GATED ? exp_d(Fm - gr.F[tj] + (double)gr.ig[tj]) : powi(pw, i - j);
+#pragma unroll 1
+    for (int c = first; c < last; ++c) o[c] = fmaf(x, value((const T*)p.v + (long)(t0 + j) * p.ldv + (long)h * Dv + c, p.v_act, 1.f), o[c]);
   }
 }
 

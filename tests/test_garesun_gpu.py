@@ -302,6 +302,43 @@ def test_a_workspace_changes_no_recurrence(gated, rot, q_act, decays):
         assert (got - want).abs().max() <= want.abs().max() * 2.0 ** -18
 
 
+@pytest.mark.parametrize("gated,rot", [(0, 0), (0, 20), (1, 0)])
+def test_values_that_are_not_finite_stay_with_later_tokens(gated, rot):
+    """an infinity and a NaN among the values of a prompt: the read-outs of the tokens before them, and of the columns beside them, are what they are without
+    them (sums of another order within 16 tokens: 2^-20 of the largest); what follows is not finite in those columns"""
+    from mlx_vlm_amd import _lib, ops
+
+    g, T, Hh, D, Dv = torch.Generator().manual_seed(rot), 200, 2, 32, 40
+    C = Dv + gated
+    q, k = (torch.randn(T, Hh * D, generator=g).bfloat16().cuda() for _ in range(2))
+    v, gate = (torch.randn(T, Hh * Dv, generator=g).bfloat16().cuda() for _ in range(2))
+    pre, bias, decay = torch.randn(2, T, Hh, generator=g).bfloat16().cuda(), torch.ones(Hh).bfloat16().cuda(), torch.tensor([0.9, 0.99]).cuda()
+    inv, tab, ws = torch.tensor([1e4 ** (-2 * i / 20) for i in range(10)]).cuda(), torch.tensor([0, T, 0, 0], dtype=torch.int32).cuda(), torch.empty(1 << 20, device="cuda")
+
+    def run(v):
+        state, ms, mtok, mprev = torch.zeros(1, Hh, D, C, device="cuda"), torch.zeros(1, Hh, device="cuda"), torch.empty(T, Hh, device="cuda"), torch.empty(1, Hh, device="cuda")
+        raw, out = torch.empty(T, Hh, C, device="cuda"), torch.empty(T, Hh * Dv, dtype=torch.bfloat16, device="cuda")
+        a = _lib.RecurrenceArgs()
+        a.q, a.k, a.v, a.g, a.ldq, a.ldk, a.ldv, a.ldg, a.ldo = q.data_ptr(), k.data_ptr(), v.data_ptr(), gate.data_ptr(), Hh * D, Hh * D, Hh * Dv, Hh * Dv, Hh * Dv
+        a.qscale, a.kscale, a.eps, a.gate_act, a.gated, a.rot_dims, a.decay, a.inv_freq = 0.5, 0.25, 1e-5, 1, gated, rot, decay.data_ptr(), inv.data_ptr()
+        a.ipre, a.fpre, a.ldi, a.ldf, a.ib, a.fb, a.cap = pre[0].data_ptr(), pre[1].data_ptr(), Hh, Hh, bias.data_ptr(), bias.data_ptr(), 12.0
+        a.mstate, a.mtok, a.mprev = ms.data_ptr(), mtok.data_ptr(), mprev.data_ptr()
+        a.seg_start, a.seg_slot, a.seg_pos0 = tab.data_ptr(), tab[2:].data_ptr(), tab[3:].data_ptr()
+        a.state, a.raw, a.out, a.H, a.D, a.Dv, a.ws, a.ws_floats = state.data_ptr(), raw.data_ptr(), out.data_ptr(), Hh, D, Dv, ws.data_ptr(), ws.numel()
+        ops.linear_recurrence(a, 1, T, False)
+        torch.cuda.synchronize()
+        return raw.cpu()
+
+    want, bad = run(v), v.clone()
+    bad[75, 3], bad[75, 39], bad[137, 7] = float("inf"), float("nan"), float("-inf")          # head 0, columns 3 and 39, then 7
+    got = run(bad)
+    close = lambda x, y: bool(((x - y).abs() <= want.abs().max() * 2.0 ** -20).all())          # noqa: E731
+    for col, first in ((3, 75), (39, 75), (7, 137)):
+        assert close(got[:first, 0, col], want[:first, 0, col]) and not torch.isfinite(got[first:, 0, col]).any()
+    rest = [c for c in range(C) if c not in (3, 39, 7)]
+    assert close(got[:, 0, rest], want[:, 0, rest]) and close(got[:, 1], want[:, 1])
+
+
 def test_one_workspace_serves_all_recurrent_layers(tmp_path):
     """a prompt over four recurrent layers of two kinds: what the step holds on to has one workspace, as large as the neediest layer's"""
     cfg = H.config([H.layer("retention"), H.layer("mlstm"), H.layer("retention", heads=2, dim=40), H.layer("mlstm")])
