@@ -860,3 +860,21 @@ def test_more_experts_than_the_plan_takes(tmp_path, family, experts):
         lm.GROUPED_SIZE = size
         got.append(_whole(lm, _ids(40, cfg["vocab"], 3)))
     assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 8])
+def test_decode_rows_at_a_checkpoint_s_width_row_by_row(tmp_path, rows):
+    """steps of 1 to 8 rows over projections as wide as a real model's (what the kernels of few rows, the split K and the matrix-core attention are chosen by),
+    every row of logits against float64: four in five within the rounding of a 16-bit chain (a router's near tie moves a row by itself, not its neighbours)"""
+    moe = dict(experts=8, top=2, ff=512, shared_ff=512)
+    cfg = H.config([H.layer("mlstm", heads=12, dim=128, vdim=128, **moe), H.layer("latent_attention", heads=12, dim=128, rot_dim=64, vdim=128, kv_rank=512, **moe),
+                    H.layer("retention", heads=12, dim=128, vdim=128, rot_dims=128, **moe)], vocab=512, width=1536)
+    W = H.weights(cfg)
+    lm = _load(tmp_path, cfg, W, "bfloat16", seqs=rows + 1)
+    lm = getattr(lm, "language_model", lm)
+    steps, texts = 4, [_ids(20 + 9 * r + 4, cfg["vocab"], r) for r in range(rows)]
+    want = torch.stack([O.Oracle(cfg, W, F64).forward(t)[-steps:] for t in texts], 1)
+    caches = [lm.make_cache() for _ in texts]
+    lm.step([(c[0]._seq, t[:-steps]) for c, t in zip(caches, texts)])
+    got = torch.stack([lm.step([(c[0]._seq, t[len(t) - steps + i: len(t) - steps + i + 1]) for c, t in zip(caches, texts)]).cpu() for i in range(steps)])
+    assert H.rel_rms(got.view(-1, cfg["vocab"]), want.reshape(-1, cfg["vocab"]), 0.8) < TOL["bfloat16"]

@@ -722,3 +722,21 @@ def test_sampled_generation_uses_the_device_sampler_and_refuses_what_is_not_buil
     with pytest.raises(NotImplementedError):
         list(generate_step(p[None], model, None, None, max_tokens=4, repetition_penalty=1.3))
     assert len(model.language_model.pool._free_seqs) == 4           # every generation gave its slot back
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 8])
+def test_decode_rows_at_a_checkpoint_s_width_row_by_row(tmp_path, rows):
+    """steps of 1 to 8 rows over projections as wide as a real model's (what the kernels of few rows, the split K and the matrix-core attention are chosen by),
+    every row of logits against float64: four in five within the rounding of a 16-bit chain (a router's near tie moves a row by itself, not its neighbours)"""
+    cfg = H.config([H.latent(heads=12, dim=128, rot_dim=64, vdim=128, kv_rank=512, scale=192 ** -0.5, window=40, mlp=H.moe(experts=8, top=2, groups=4, keep=2, ff=640)),
+                    H.attention(heads=12, kv_heads=2, dim=128, vdim=128, scale=128 ** -0.5, softcap=30.0, mlp=H.moe(experts=8, top=2, groups=4, keep=2, ff=640))],
+                   vocab=512, width=1536)
+    W = H.weights(cfg)
+    lm = _load(tmp_path, cfg, W, "bfloat16", seqs=rows + 1)
+    lm = getattr(lm, "language_model", lm)
+    orc, steps, texts = O.Oracle(cfg, W, F64), 4, [_ids(20 + 9 * r + 4, cfg["vocab"], r) for r in range(rows)]
+    want = torch.stack([orc.forward(t)[-steps:] for t in texts], 1)
+    caches = [lm.make_cache() for _ in texts]
+    lm.step([(c[0]._seq, t[:-steps]) for c, t in zip(caches, texts)])
+    got = torch.stack([lm.step([(c[0]._seq, t[len(t) - steps + i: len(t) - steps + i + 1]) for c, t in zip(caches, texts)]).cpu() for i in range(steps)])
+    assert H.rel_rms(got.view(-1, cfg["vocab"]), want.reshape(-1, cfg["vocab"]), 0.8) < TOL["bfloat16"]
