@@ -22,7 +22,7 @@ struct RowsArgs {
   long lda, ldw, ldc, sA, sW, sC;
 };
 
-template <typename TA, typename TC, int MT, int NT, int U>
+template <typename TA, typename TC, int MT, int NT, int U, bool TURNS = false>
 __global__ __launch_bounds__(256) void linear_rows_mfma_kernel(RowsArgs p) {
   constexpr int PITCH = 20, WAVES = 4, AV = sizeof(TA) == 2 ? 2 : 4, PER = 16 / AV;          // 16-byte pieces of a lane's 16 activations
   __shared__ __align__(16) float red[WAVES][NT * MT][16 * PITCH];
@@ -82,8 +82,8 @@ __global__ __launch_bounds__(256) void linear_rows_mfma_kernel(RowsArgs p) {
       }
     }
     // short chains on the matrix unit, added up by rounding additions: long ones round worse (router logits of 8 rows, K = 1536: relative error
-    // 1.3e-7 in one chain a wave, 7e-8 so).  The U pieces of a turn are added to each other first (K = 17920, 2 rows: 1.67e-7 one by one,
-    // 1.06e-7 so)
+    // 1.3e-7 in one chain a wave, 7e-8 so).  TURNS, fp32 results of up to 8 rows: the U pieces of a turn are added to each other first, which is as close as
+    // vlm_linear_rows_bf16w or closer (K = 4096 / 17920: 9.5e-8 / 1.67e-7 one by one, 7.95e-8 / 1.07e-7 so, 8.3e-8 / 1.30e-7 there)
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
     f32x4_t turn[NT][MT];
 #pragma unroll
@@ -106,8 +106,12 @@ __global__ __launch_bounds__(256) void linear_rows_mfma_kernel(RowsArgs p) {
             }
             t[0] = (t[0] + t[1]) + (t[2] + t[3]);
           }
-          turn[j][i] = u ? turn[j][i] + t[0] : t[0];
-          if (u == U - 1) acc[j][i] += turn[j][i];
+          if constexpr (TURNS) {
+            turn[j][i] = u ? turn[j][i] + t[0] : t[0];
+            if (u == U - 1) acc[j][i] += turn[j][i];
+          } else {
+            acc[j][i] += t[0];
+          }
         }
   }
 #pragma unroll
@@ -136,6 +140,12 @@ void launch_rows(RowsArgs a, int batch, hipStream_t st) {
   a.R = (int)std::min<long>(16, (all + 256 * nt - 1) / (256 * nt));
   const dim3 grid((a.N + a.R * nt - 1) / (a.R * nt), batch), block(256);
   constexpr bool f = sizeof(TA) == 4;
+  if constexpr (!f && sizeof(TC) == 4)
+    if (a.M <= 8) {
+      if (nt == 1) hipLaunchKernelGGL((linear_rows_mfma_kernel<TA, TC, 1, 1, 4, true>), grid, block, 0, st, a);
+      else hipLaunchKernelGGL((linear_rows_mfma_kernel<TA, TC, 1, 2, 3, true>), grid, block, 0, st, a);
+      return;
+    }
   if (a.M > 32) {                                                    // (few columns: blocks of 16 rows fill the chip)
     a.R = std::min(16, a.N);
     hipLaunchKernelGGL((linear_rows_mfma_kernel<TA, TC, 1, 1, f ? 3 : 4>), dim3((a.N + a.R - 1) / a.R, batch, (a.M + 15) / 16), block, 0, st, a);
@@ -160,7 +170,7 @@ VLM_INTERNAL int vlm_linear_rows_mfma_try(const void* A, const void* W, void* C,
   // more rows over few columns, as blocks of 16: router logits [8, 1536] of 2048 rows 29 -> 7.5 us
   if (M > 32 ? N > 64 || batch > 1 || M > 65535 * 16 : false) return -1;
   const bool fits = (long)N * batch <= 8192 || (M <= 8 && (long)N * batch * K <= 4 << 20);
-  if (!fits || (K > 4096 && !(accumulate && M <= 8)) || K % 8 || lda % va || sA % va || ldw % 8 || sW % 8 || (((uintptr_t)A | (uintptr_t)W) & 15)) return -1;
+  if (!fits || (K > 4096 && !(accumulate && !a_f32 && M <= 8)) || K % 8 || lda % va || sA % va || ldw % 8 || sW % 8 || (((uintptr_t)A | (uintptr_t)W) & 15)) return -1;
   const RowsArgs a{A, (const bf16_t*)W, C, M, N, K, 0, accumulate, lda, ldw, ldc, sA, sW, sC};
   hipStream_t st = (hipStream_t)stream;
   if (a_f32) c_f32 ? launch_rows<float, float>(a, batch, st) : launch_rows<float, bf16_t>(a, batch, st);

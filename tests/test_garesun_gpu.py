@@ -699,6 +699,23 @@ def test_linear_any_few_rows_over_bf16_weights(M, N, K, batch):
                 assert over.max() <= 0, (ta, tc, add)
 
 
+@pytest.mark.parametrize("N,K,add", [(64, 3584, False), (1536, 4096, True), (6144, 3000, True), (1536, 17920, True)])
+def test_fp32_results_of_few_rows_are_as_close_as_the_streaming_form_s(N, K, add):
+    """distance to float64 over 2, 4 and 8 rows of several draws (some 10^4 sums: the mean square is known to a few parts in a hundred): no larger than that of the
+    kernel that takes such rows otherwise"""
+    from mlx_vlm_amd import ops
+
+    g, e = torch.Generator(device="cuda").manual_seed(K), [0.0, 0.0]
+    for M in (2, 4, 8) * (8 if N < 1000 else 1):
+        a, w = (torch.randn(n, K, generator=g, device="cuda").bfloat16() for n in (M, N))
+        ref = a.double() @ w.double().T
+        for i, f in enumerate((ops.linear_any, ops.linear_rows_bf16w)):
+            x = torch.zeros(M, N, device="cuda")
+            f(a, w, out=x, accumulate=add)
+            e[i] += (x.double() - ref).pow(2).sum().item()
+    assert e[0] <= 1.05 * e[1], e
+
+
 @pytest.mark.parametrize("experts", [6, 36])
 @pytest.mark.parametrize("rows", [1, 2, 3, 4])
 def test_steps_of_few_rows_sum_onto_the_stream_in_fp32(tmp_path, rows, experts):
