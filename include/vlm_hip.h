@@ -55,6 +55,9 @@ int vlm_abi_version(void);
  * K % 8 == 0, N % 8 == 0.  With VLM_EPI_SWIGLU, C is [M, N/2]. */
 int vlm_gemm_bf16(const void* A, const void* W, const void* bias, const void* res, void* C, int M, int N, int K,
                   int lda, int ldw, int ldc, int ldres, int epilogue, void* stream);
+/* The same without bias and residual, and with room for split-K partials (8 * M * N fp32 values serve every choice the rule makes) that the caller
+ * keeps until the product is done: a capture, where the library allocates none, splits K as an eager call does */
+int vlm_gemm_bf16_ws(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, void* ws, long ws_bytes, void* stream);
 
 /* The qkv projection of the vision attention with apply_rotary_pos_emb_vision (vision.py:35-50,141-142) as its epilogue:
  * C = rope2d(A . W^T + bias) on the first rope_cols columns (the q and k heads, head_dim wide), plain bias on the rest.
@@ -62,9 +65,6 @@ int vlm_gemm_bf16(const void* A, const void* W, const void* bias, const void* re
  * h * head_dim + 2 d + 1 (q.k is invariant under a common permutation of the head dimension) - so that a rotation pair
  * is two adjacent outputs.  cos_sin: fp32 [2][M][head_dim / 2]: cos rows then sin rows of VisionModel.rot_pos_emb
  * (vision.py:219-255).  Rounding as the reference: bf16(linear + bias), fp32 rotation, one rounding. */
-/* the same without bias and residual, and with room for split-K partials (8 * M * N fp32 values serve every choice the rule makes) that the caller
- * keeps until the product is done: a capture, where the library allocates none, splits K as an eager call does */
-int vlm_gemm_bf16_ws(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, void* ws, long ws_bytes, void* stream);
 int vlm_gemm_bf16_rope2d(const void* A, const void* W, const void* bias, const void* cos_sin, void* C, int M, int N, int K,
                          int lda, int ldw, int ldc, int head_dim, int rope_cols, void* stream);
 

@@ -2,13 +2,14 @@
 //
 //     C[b][m][n] (+)= sum_k A[b][m][k] * W[b][n][k]          b < batch, any M, N, K, any leading dimension
 //
-// A, W and C are each bf16 or fp32 (codes 0 / 1); products and sums are fp32 on v_mfma_f32_16x16x4_f32 (linear_f32_mfma_kernel: an output
-// is eight chains over fixed pieces of k, added in a fixed order), so a row of C depends on
-// nothing but its own row of A: the result of a token is the same bits whatever else is in the batch and however a
-// prompt was cut into steps.  With all three in fp32 this is the true 32-bit product of the float32 serving mode; with
-// fp32 C and `accumulate` it adds a projection straight onto an fp32 residual stream.
+// A, W and C are each bf16 or fp32 (codes 0 / 1).  A product with an fp32 operand is fp32 throughout, on v_mfma_f32_16x16x4_f32 (linear_f32_ranges_kernel and
+// linear_f32_tiles_kernel: an output is eight chains over fixed pieces of k, added in a fixed order).  With all three in fp32 - the true 32-bit product of
+// the float32 serving mode - that holds for every number of rows, so a row of C depends on nothing but its own row of A: the result of a token is the same
+// bits whatever else is in the batch and however a prompt was cut into steps.  With bf16 weights the number of rows chooses the kernel (few rows:
+// linear_rows_kernel and linear_rows_mfma.hip), and with it the order of the sums.  fp32 C and `accumulate` add a projection straight onto an fp32
+// residual stream.
 //
-// bf16 A and W with aligned rows and more than 8 rows of A take the bf16 matrix cores instead (linear_any_mfma_kernel: fp32 sums in blocks of 32 k).
+// bf16 A and W with aligned rows and more than 8 rows of A take the bf16 matrix cores (linear_any_mfma_kernel: fp32 sums in blocks of 32 k).
 //
 // Per-head projections of one tensor (latent attention's absorbed key / value maps) run as `batch` with element strides between heads.
 #include "common.hpp"

@@ -3,8 +3,9 @@
 One `step()` runs any number of segments, each a run of consecutive tokens of one sequence - a whole prompt, a portion of
 one, or a single decoded token - side by side.  The host builds ONE int32 table per step (token -> sequence slot / position,
 segment -> slot / first position, query blocks, wanted rows) and every kernel indexes through it, so a prompt portion next
-to decode rows is one launch sequence and the result of a token does not depend on how its prompt was cut or on its
-neighbours in the batch.  `prefill`, `decode_begin` / `decode_run` and `decode_step_rows` are the entry points the
+to decode rows is one launch sequence.  In float32 serving the result of a token is the same bits however its prompt was
+cut and whatever its neighbours in the batch are; in bfloat16 the size of a step chooses kernels and splits, and with them
+the order of fp32 sums.  `prefill`, `decode_begin` / `decode_run` and `decode_step_rows` are the entry points the
 generation paths (generate.py, batch.py) call on every language model; here they are thin wrappers over `step()`.
 
 A model derives from RaggedLanguageModel and brings `load_weights` (which also builds `self.pool`, a HybridPool),
