@@ -25,7 +25,8 @@
 //         multiplier per head, a cap (cap tanh(s / cap)), a gate per value column, a term exp(0) in the denominator.  Against the scalar
 //         kernels of window_attn.hip (us): 1500 tokens of 12 heads (2 key heads) of 128, window 1024: 505 -> 81; 2048 tokens, no window, cap:
 //         1210 -> 165; 1100 tokens of 28 heads (4): 708 -> 147; 40 tokens 19 -> 20; 8 decode rows over 700 keys 19 -> 17, one over 16000 keys
-//         606 -> 28, over 20 keys 11.8 -> 12.5.  Bound by the loads of keys and values from L2, which every two heads and 16 queries read anew.
+//         606 -> 28.  Over 20 keys the scalar kernel is ahead (5.6 | 11.6; of 256 columns 6.6 | 20): contexts that are known to stay
+//         short keep it (ROW_KEYS of ops.py).  Bound by the loads of keys and values from L2, which every two heads and 16 queries read anew.
 //
 // The waves (of all splits) take turns over the key tiles (16 or 32 keys at multiples of that counted from the sequence's first token) and
 // work straight from global memory in the operand layout, without LDS traffic for keys or values (see attn_mfma.hpp).  Running maximum

@@ -21,7 +21,8 @@
 //   rows (decode)    workgroup = one token x up to 16 heads, one page at a time through LDS: the waves share the page's keys for the scores,
 //                    exchange them, and share the value columns for the read-out; `nsplit` workgroups take turns over the pages, a second
 //                    kernel merges their results.  fp32 queries: 8 rows of 12 heads over 700 keys 45 -> 20 us, one row over 16384 keys
-//                    1476 -> 41 us, over 20 keys 11.5 -> 13.6 us (the merge; a captured step cannot know how few the keys are).
+//                    1476 -> 41 us.  Over 20 keys the scalar kernel is ahead (7.3 | 16.1 us, R = 128 5.2 | 9.3; 512 keys 34 | 16 and 14 | 9.6):
+//                    contexts that are known to stay short keep it (ROW_KEYS of ops.py).
 #include "common.hpp"
 #include "../../include/vlm_hip.h"
 #include "recurrence_finish.hpp"

@@ -179,7 +179,8 @@ class LanguageModel(RaggedLanguageModel):
             ops.window_attn_blocks(q, kpool, vpool, pl.qb_start, pl.qb_count, pl.tok_seq, pl.tok_pos, pool.block_table, H, G, D, Dv,
                                    ns.scale, out, **args)
         else:
-            ops.window_attn_rows(q, kpool, vpool, pl.tok_seq, pl.tok_pos, pool.block_table, H, G, D, Dv, ns.scale, out, **args)
+            ops.window_attn_rows(q, kpool, vpool, pl.tok_seq, pl.tok_pos, pool.block_table, H, G, D, Dv, ns.scale, out, keys=pl.keys,
+                                 **args)
         keep.append(q)
         return out
 

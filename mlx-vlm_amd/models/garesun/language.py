@@ -211,7 +211,7 @@ class LanguageModel(RaggedLanguageModel):
                                                 bt, H, R, Dr, ns.scale, gate=col("g"))
                 else:
                     ol = ops.latent_attn(qabs.view(Tn, H, R + Dr), pool.rows[ns.src], tok_seq_d, tok_pos_d, bt, H, R, Dr, ns.scale,
-                                         gate=col("g"))
+                                         gate=col("g"), keys=pl.keys)
                 ops.linear_any(ol.view(Tn, H * R), ns.uv.view(H * Dv, R), out=cat, M=Tn, N=Dv, K=R, batch=H, stride_a=R, stride_w=Dv * R,
                                stride_c=Dv)
                 keep += [qabs, ol]

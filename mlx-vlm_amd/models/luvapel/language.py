@@ -203,7 +203,7 @@ class LanguageModel(RaggedLanguageModel):
                                    ns.scale, out, temp=ns.temp, window=ns.window, gate=col("lg"))
         else:
             ops.window_attn_rows(q, kpool, vpool, pl.tok_seq, pl.tok_pos, pool.block_table, H, G, D, D, ns.scale, out, temp=ns.temp,
-                                 window=ns.window, gate=col("lg"))
+                                 window=ns.window, gate=col("lg"), keys=pl.keys)
         keep.append(q)
         return out
 

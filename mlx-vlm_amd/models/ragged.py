@@ -25,7 +25,7 @@ import torch
 
 from .. import _lib, ops
 from .base import LanguageModelOutput
-from .cache import HybridPool, PagedSequence
+from .cache import PAGE, HybridPool, PagedSequence
 
 
 def _al8(n: int) -> int:
@@ -234,7 +234,13 @@ class RaggedLanguageModel:
                                .reshape(-1).to(torch.int32) for _, ids in entries])
         return SimpleNamespace(seqs=seqs, lens=lens, nseg=nseg, Tn=Tn, rows=rows, all_rows=bool(rows.size == Tn and np.array_equal(rows, np.arange(Tn))),
                                tok_seq=parts[0], tok_pos=parts[1], cu=parts[2], slot=parts[3], pos0=parts[4], rows_d=parts[5], qb_start=parts[6],
-                               qb_count=parts[7], ids=ids_d, md=md)
+                               qb_count=parts[7], ids=ids_d, md=md, keys=self._keys(seqs))
+
+    @staticmethod
+    def _keys(seqs):
+        """the most tokens that the pages reserved for any of these sequences hold: generation reserves what a request may grow to before
+        its first step, so that this says, steadily over its steps, how long its context can get"""
+        return max(len(s.pages) for s in seqs) * PAGE
 
     _trace = None      # a list: step() appends the stream after every layer (debugging / tests)
 
@@ -285,10 +291,13 @@ class RaggedLanguageModel:
         token written back as the next input.  With use_graph the launch sequence of a (state, row count, sampler) is captured
         into a HIP graph the second time it runs and replayed from then on: the host then only reserves pages and refills the
         small table of (sequence slot, position) per row - a step is ~100 launches, which the host cannot issue as fast as the
-        GPU runs them."""
+        GPU runs them.  The key holds the class of the rows' reserved contexts too, by which the attention of the step takes its
+        kernels (a graph computes the right result at any context; the class is a matter of speed)."""
         n = len(seqs)
+        for s in seqs:
+            s.reserve(s.offset + 1)
         entries = [(s, st.tok[r:r + 1]) for r, s in enumerate(seqs)]
-        key = (id(st), n, bool(with_logprobs), tuple(sorted(sampler_args.items())))
+        key = (id(st), n, ops.row_keys(self._keys(seqs)), bool(with_logprobs), tuple(sorted(sampler_args.items())))
         ent = self._graphs.get(key) if use_graph else None
         if ent is None:
             self._rows_step(st, seqs, advance=False)

@@ -143,7 +143,8 @@ class LanguageModel(RaggedLanguageModel):
             ops.window_attn_blocks(q, kpool, vpool, pl.qb_start, pl.qb_count, pl.tok_seq, pl.tok_pos, pool.block_table, H, G, D, Dv,
                                    ns.scale, out, **args)
         else:
-            ops.window_attn_rows(q, kpool, vpool, pl.tok_seq, pl.tok_pos, pool.block_table, H, G, D, Dv, ns.scale, out, **args)
+            ops.window_attn_rows(q, kpool, vpool, pl.tok_seq, pl.tok_pos, pool.block_table, H, G, D, Dv, ns.scale, out, keys=pl.keys,
+                                 **args)
         keep.append(q)
         return out
 
@@ -165,7 +166,8 @@ class LanguageModel(RaggedLanguageModel):
             ol = ops.latent_attn_blocks(qabs.view(Tn, H, R + Dr), cpool, pl.qb_start, pl.qb_count, pl.tok_seq, pl.tok_pos, bt, H, R, Dr,
                                         ns.scale, window=ns.window)
         else:
-            ol = ops.latent_attn(qabs.view(Tn, H, R + Dr), cpool, pl.tok_seq, pl.tok_pos, bt, H, R, Dr, ns.scale, window=ns.window)
+            ol = ops.latent_attn(qabs.view(Tn, H, R + Dr), cpool, pl.tok_seq, pl.tok_pos, bt, H, R, Dr, ns.scale, window=ns.window,
+                                 keys=pl.keys)
         out = torch.empty(Tn, _al8(H * Dv), dtype=self.dtype, device=dev)[:, : H * Dv]
         ops.linear_any(ol.view(Tn, H * R), ns.uv.view(H * Dv, R), out=out, M=Tn, N=Dv, K=R, batch=H, stride_a=R, stride_w=Dv * R, stride_c=Dv)
         ops.glu_rows(col("g"), out, ops.GLU_SIGMOID, out=out)

@@ -699,15 +699,40 @@ def _sink_ok(sink, H):
         raise _lib.VlmHipError("attention: fp32 sinks, one per head, expected")
 
 
-def latent_attn(q, pool, tok_seq, tok_pos, block_table, H, R, Dr, scale, gate=None, out=None, window=0, sink=None):
+# Decode rows over few keys run on the scalar kernels, over more on the matrix cores, whose workgroups stage tiles of 32 keys and split a long
+# context among them, which a short one pays for as well.  Their lines cross, in us (1 to 8 rows, 4 to 28 heads, scalar / matrix cores):
+#   keys                20          128         256         384         512
+#   latent R + Dr  128   5.1 /  8.9   5.9 /  9.0   7.7 /  9.2   9.5 /  9.2  11.2 /  9.3
+#                  192   5.3 /  9.6   6.8 /  9.6   9.4 /  9.6  11.9 /  9.7  14.5 /  9.8
+#                  320   6.0 / 11.8   8.6 / 11.8  12.7 / 11.8  17.0 / 11.9  21.0 / 11.9
+#                  576   7.3 / 16.5  12.3 / 16.6  19.6 / 16.6  27.0 / 16.8  34.3 / 17.0
+#   windowed D      64   5.2 /  9.4   5.8 /  9.9   7.2 /  9.9   8.6 / 10.0  10.0 / 10.1
+#                  128   5.6 / 11.4   6.8 / 12.4   9.1 / 12.5  11.6 / 12.6  13.9 / 12.6
+#                  256   6.6 / 20.1   8.9 / 20.2  13.3 / 20.3  18.0 / 20.2  22.3 / 20.4
+# A caller that knows how many keys its rows can ever see says so in `keys`.  A context grows up to that bound, so the lines are not where the
+# times at the bound meet but where their means on the way there do.
+ROW_KEYS = (256, 384)
+
+
+def row_keys(keys):
+    """the class of a bound on the keys of decode rows: bounds of one class take the same kernels (None: no bound that matters)"""
+    return next((k for k in ROW_KEYS if keys is not None and keys <= k), None)
+
+
+def _few_keys(keys, window, line):
+    return keys is not None and (min(keys, window) if window > 0 else keys) <= line
+
+
+def latent_attn(q, pool, tok_seq, tok_pos, block_table, H, R, Dr, scale, gate=None, out=None, window=0, sink=None, keys=None):
     """q fp32 [T, H, R + Dr] over the latent pool -> fp32 [T, H, R] (times sigmoid(gate[t, h]) when given); window > 0: a query
-    reaches back window - 1 tokens; sink fp32 [H]: exp(sink[h]) in the softmax's denominator"""
+    reaches back window - 1 tokens; sink fp32 [H]: exp(sink[h]) in the softmax's denominator; keys: an upper bound of the keys a row's
+    context holds, where the caller knows one (it decides the kernel, see ROW_KEYS)"""
     _dev(q, pool, tok_seq, tok_pos, block_table, gate, out, sink)
     _sink_ok(sink, H)
     T = q.shape[0]
     if out is None:
         out = torch.empty(T, H, R, dtype=torch.float32, device=q.device)
-    if 0 < T <= 65535 and _latent_f32_mfma(q, pool, H, R, Dr, gate, out):
+    if 0 < T <= 65535 and not _few_keys(keys, window, ROW_KEYS[R <= 128]) and _latent_f32_mfma(q, pool, H, R, Dr, gate, out):
         a = _latent_mfma_args(q, pool, tok_seq, tok_pos, block_table, H, R, Dr, scale, gate, out, window, sink)
         nsplit, part = _latent_row_split(a, T, block_table, window, None, q.device)
         check(_lib.lib().vlm_latent_attn_mfma_f32(C.byref(a), 0, T, _stream()), "latent_attn_mfma_f32")
@@ -1104,10 +1129,12 @@ def window_attn_blocks(q, kpool, vpool, qb_start, qb_count, tok_seq, tok_pos, bl
 
 
 def window_attn_rows(q, kpool, vpool, tok_seq, tok_pos, block_table, H, KH, D, Dv, scale, out, temp=None, window=0, gate=None, cap=0.0,
-                     gate_head=False, sink=False):
-    """decode form of the windowed attention"""
+                     gate_head=False, sink=False, keys=None):
+    """decode form of the windowed attention; keys: an upper bound of the keys a row's context holds, where the caller knows one (it decides
+    the kernel, see ROW_KEYS)"""
     _dev(q, kpool, vpool, tok_seq, tok_pos, block_table, out, temp, gate)
-    if vpool.dtype == torch.bfloat16 and D <= 320 and Dv <= 256:          # (the matrix-core form's tiles; it is measured in csrc/grouped_attn.hip)
+    # (the matrix-core form's tiles; it is measured in csrc/grouped_attn.hip)
+    if vpool.dtype == torch.bfloat16 and D <= 320 and Dv <= 256 and not _few_keys(keys, window, ROW_KEYS[1]):
         a = _lib.GroupedAttnArgs()
         a.q, a.kpool, a.vpool, a.tok_seq, a.tok_pos, a.block_table = _p(q), _p(kpool), _p(vpool), _p(tok_seq), _p(tok_pos), _p(block_table)
         a.max_pages, a.H, a.KH, a.D, a.Dv, a.scale, a.window = block_table.shape[1], int(H), int(KH), int(D), int(Dv), float(scale), int(window)

@@ -334,6 +334,40 @@ def test_latent_attention_f32_queries_over_bf16_rows(R, Dr, Hh):
         assert torch.equal(got, one[0, 0, :R].float().expand(2, Hh, R))
 
 
+@pytest.mark.parametrize("keys,window", [(64, 0), (256, 0), (257, 0), (384, 0), (385, 0), (5000, 256), (5000, 385), (None, 0)])
+def test_a_bound_on_the_keys_changes_the_kernel_and_not_the_read_out(monkeypatch, keys, window):
+    """both kernels of decode rows lie within sums of fp32 of float64 (see above), whichever a bound on the keys takes"""
+    from mlx_vlm_amd import ops
+    from mlx_vlm_amd.models.cache import PAGE
+
+    g = torch.Generator().manual_seed(5)
+    calls, bt, n = [], torch.arange(7, dtype=torch.int32).view(1, 7).cuda(), min(keys or 400, 440)
+    tok = (torch.zeros(3, dtype=torch.int32).cuda(), torch.tensor([0, n // 2, n - 1], dtype=torch.int32).cuda(), bt)
+    seen = [range(max(0, p - window + 1) if window else 0, p + 1) for p in (0, n // 2, n - 1)]
+    for name in ("_latent_row_split", "_grouped_row_split"):
+        monkeypatch.setattr(ops, name, lambda *a, real=getattr(ops, name): (calls.append(1), real(*a))[1])
+    few = None if keys is None else min(keys, window or keys)
+    for R, Dr, Hh in ((128, 64, 5), (256, 64, 3)):
+        q, pool = torch.randn(3, Hh, R + Dr, generator=g).cuda(), torch.randn(7, PAGE, R + Dr, generator=g).bfloat16().cuda()
+        calls.clear()
+        got = ops.latent_attn(q, pool, *tok, Hh, R, Dr, (R + Dr) ** -0.5, window=window, keys=keys)
+        assert bool(calls) == (few is None or few > (384 if R <= 128 else 256))
+        flat = pool.view(-1, R + Dr).double()
+        want = torch.stack([torch.softmax(q[t].double() @ flat[s].T * (R + Dr) ** -0.5, -1) @ flat[s, :R] for t, s in enumerate(map(list, seen))])
+        assert float((got.double() - want).abs().max()) <= 2 ** -23 * 2 * (R + Dr + n) / 100 * float(want.abs().max())
+    for D, Dv, KH in ((128, 128, 2), (40, 24, 1)):
+        q, kpool, vpool = torch.randn(3, 4 * D, generator=g).cuda(), torch.randn(7, PAGE, KH * D, generator=g).cuda(), torch.randn(7, PAGE, KH * Dv, generator=g).bfloat16().cuda()
+        out = torch.empty(3, 4 * Dv, dtype=torch.bfloat16, device="cuda")
+        calls.clear()
+        ops.window_attn_rows(q, kpool, vpool, *tok, 4, KH, D, Dv, D ** -0.5, out, window=window, keys=keys)
+        assert bool(calls) == (few is None or few > 384)
+        for t, s in enumerate(map(list, seen)):
+            k, v = (x.view(-1, KH, w)[s].double().repeat_interleave(4 // KH, 1).transpose(0, 1).contiguous() for x, w in ((kpool, D), (vpool, Dv)))
+            w8 = torch.softmax((q[t].double().view(4, 1, D) * k).sum(-1) * D ** -0.5, -1)
+            want = (w8[..., None] * v).sum(1)
+            assert bool(((out[t].double().view(4, Dv) - want).abs() <= want.abs() * 2.0 ** -8 + 2 ** -23 * 2 * (D + n) / 100 * float(want.abs().max())).all())
+
+
 def test_latent_rows_and_query_parts_rotate_half():
     from mlx_vlm_amd import ops
     from mlx_vlm_amd.models.cache import PAGE
@@ -709,6 +743,43 @@ def test_captured_decode_steps_equal_eager_ones(tmp_path):
     assert any(isinstance(v, tuple) for v in lm._graphs.values())            # a graph was captured and used
     for i, ((t0, l0), (t1, l1)) in enumerate(zip(eager, graph)):
         assert torch.equal(t0, t1) and torch.equal(l0, l1), i
+
+
+@pytest.mark.parametrize("prompt,kind", [(250, "latent"), (378, "window")])
+def test_decode_rows_of_short_contexts_take_the_scalar_kernels(tmp_path, monkeypatch, prompt, kind):
+    """what a request has reserved decides: up to 256 keys (384 for windowed rows) the scalar kernel, past them the matrix cores.  A request that
+    outgrows its reservation moves from one to the other, in eager and in captured steps with the same bits"""
+    from mlx_vlm_amd import ops
+    from mlx_vlm_amd.sample_utils import make_sampler
+
+    layer = H.latent(kv_rank=136, window=0, mlp="dense") if kind == "latent" else H.attention(window=0)
+    cfg = H.config([layer])
+    W = H.weights(cfg, seed=3)
+    lm = _load(tmp_path, cfg, W, "bfloat16", tokens=2048, seqs=4).language_model
+    calls, name = [], "_latent_row_split" if kind == "latent" else "_grouped_row_split"
+    real = getattr(ops, name)
+    monkeypatch.setattr(ops, name, lambda *a: (calls.append(1), real(*a))[1])
+    text, line = _ids(prompt, cfg["vocab"], 9), 256 if kind == "latent" else 384
+
+    def run(use_graph):
+        caches = lm.make_cache_batch(1)
+        lg = lm.prefill(torch.as_tensor(text).cuda().reshape(-1, 1), None, caches, [prompt])
+        st = lm.decode_begin(caches, lg.argmax(-1), np.zeros((1, 1)), max_new_tokens=3)
+        out, mfma = [int(lg.argmax(-1))], []
+        for i in range(14):
+            calls.clear()
+            lm.decode_run(st, 1, make_sampler().engine_args(), use_graph=use_graph)
+            out.append((st.logits.float().cpu()[0], int(st.tok[0])))
+            mfma.append(len(calls))
+        caches[0][0]._seq.release()
+        return out, mfma
+    (eager, mfma), (graph, _) = run(False), run(True)
+    # the step that feeds the token of position p sees p + 1 keys; the pages reserved for it hold at most `line` up to there
+    assert [bool(n) for n in mfma] == [prompt + i + 1 > line for i in range(14)]
+    assert eager[0] == graph[0] and all(torch.equal(a[0], b[0]) and a[1] == b[1] for a, b in zip(eager[1:], graph[1:]))
+    fed = np.concatenate([text, [eager[0]], [t for _, t in eager[1:-1]]]).astype(np.int32)
+    want = O.Oracle(cfg, W, F64).forward(fed)[-14:]
+    assert H.rel_rms(torch.stack([l for l, _ in eager[1:]]), want) < TOL["bfloat16"]
 
 
 def test_sampled_generation_uses_the_device_sampler_and_refuses_what_is_not_built(tmp_path):
