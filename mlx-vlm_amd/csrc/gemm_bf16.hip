@@ -53,7 +53,7 @@ __device__ __forceinline__ int lds_off(int row, int slot) { return row * ROWB + 
 // INTO LDS: a thread's 16-byte LDS chunk (8 consecutive k of one row) is exactly one q word, and BK = 64 = the group
 // size, so a K tile of a row has ONE (scale, bias).  The LDS image is bit for bit the one the bf16 kernel builds from
 // vlm_dequant_w4's output (same fp32 scale * q + bias, one rounding: mx.dequantize), so the fused GEMM equals
-// dequantise-then-GEMM bit for bit while reading 4.5 instead of 16 + 16 + 16 bits per weight (nn.QuantizedLinear /
+// dequantise-then-GEMM bit for bit wherever both split K alike, while reading 4.5 instead of 16 + 16 + 16 bits per weight (nn.QuantizedLinear /
 // mx.quantized_matmul at L > 1, reference utils.py:918-967).
 // LDS stages of the LDS-DMA K loop per tile shape (2 = the plain double buffer) and the counted wait it needs
 template <int BM, int BN>
@@ -687,13 +687,48 @@ VLM_INTERNAL void vlm_gemm_splitk_unshare(void* to) {
 
 namespace {
 
+// What a product by tiles of 64 x 64, 64 x 128 (three stages up to two workgroups a compute unit, two from there) or 128 x 128 takes in us: a
+// launch, the K tiles of a workgroup times what one takes with that many workgroups on the busiest compute unit, the partials there and back.
+// Fitted to 176 products of 65 to 3000 rows (N 512 to 5120, K 4096 to 24576) by every form: half of them within 4 %.
+double tiles_us(int tm, int tn, long tiles, int splits, int M, int N, int K) {
+  const long n = (tiles * splits + 255) / 256;
+  const double k_tile = tn == 64   ? 0.175 * n                                                             // (the loads from L2 bound it)
+                        : tm == 64 ? 0.775 * (n / 3) + (n % 3 == 0 ? 0. : n % 3 == 1 ? 0.35 : 0.53)
+                                   : 0.76 * (n / 2) + (n % 2 == 0 ? 0. : 0.60);
+  return 8. + k_tile * K / (64. * splits) + (splits > 1 ? 1.3e-6 * splits * M * N : 0.);
+}
+
 // Split-K on 128-column tiles, for the long-K products of prompts and images (more than 64 rows, K >= 4096) whose tiles leave compute units without
-// work.  -> splits (0: not), bm = 128 or 64 rows a tile.  The estimate that it takes the least of: flops at 900 (128 x 128) or 700 (64 x 128)
-// TFLOP/s times how full the last round of 512 workgroups is, and the partials there and back at 9 TB/s (they stay in the last-level cache).
-// Measured, us (single pass as chosen below | 64 x 64 in 3 | chosen here): 1486 x 1536 x 8960 87 | - | 55 (128, 3); 1020 x 1280 x 5120 47 | - | 27 (64, 3);
-// 700 x 1536 x 8960 92 | 42 (64 x 64 in 8) | 36 (128, 6); 2048 x 1280 x 5120 58 | - | 41 (128, 3); 386 x 1536 x 8960 - | 26 | 26 (64, 6);
-// 1503 x 3584 x 18944 235 | - | 215 (128, 3).  At K = 4736 and 336 tiles the single pass is ahead (60 and 73), with few tiles of 64 x 64 the rule below.
+// work.  -> splits (0: not), bm = 128 or 64 rows a tile: the form whose estimate is a tenth below that of what the rules of launch_epi take.
+// Measured, us (launch_epi's form | chosen here): 1486 x 1536 x 8960 80 | 53 (128, 3); 1020 x 1280 x 5120 34 | 27 (64, 3); 700 x 1536 x 8960 48 | 36
+// (128, 6); 2048 x 1280 x 5120 50 | 40 (128, 3); 386 x 1536 x 8960 32 | 27 (64, 6); 1486 x 3584 x 18944 230 | 210 (128, 3).  Not taken, us (launch_epi's |
+// best split): 386 x 4096 x 4096 23 | 27; 2048 x 1024 x 4096 27 | 29; 2048 x 3072 x 24576 313 | 382.  Of the 176 products one loses (386 x 2560 x 6912
+// 29 | 31); they take 0.908 of their time without splits here.
 int wide_split(int M, int N, int K, int& bm) {
+  const long t128 = (long)vlm_cdiv(M, 128) * vlm_cdiv(N, 128), t64n = (long)vlm_cdiv(M, 64) * vlm_cdiv(N, 128), t64 = (long)vlm_cdiv(M, 64) * vlm_cdiv(N, 64);
+  if (M <= 64 || K < 4096 || t128 >= 512 || (t128 > 256 && K < 16384)) return 0;
+  double best = 0.9 * (t64 < 256                   ? tiles_us(64, 64, t64, (int)std::min<long>(8, std::max<long>(2, (512 + t64 - 1) / t64)), M, N, K)
+                       : t64 < 640 && K >= 16384   ? tiles_us(64, 64, t64, 3, M, N, K)
+                       : t128 >= 200               ? tiles_us(128, 128, t128, 1, M, N, K)
+                       : t64n >= 200 && t64 >= 768 ? tiles_us(64, 128, t64n, 1, M, N, K)
+                                                   : tiles_us(64, 64, t64, 1, M, N, K));
+  int splits = 0;
+  for (int tm = 128; tm >= 64; tm -= 64) {
+    const long t = tm == 128 ? t128 : t64n;
+    for (int s = 2; s <= 6 && K / s >= 1024; ++s) {
+      if (t * s < 384 || (size_t)s * M * N * sizeof(float) > SPLITK_WS_BYTES) continue;
+      const double us = tiles_us(tm, 128, t, s, M, N, K);
+      if (us < best) best = us, splits = s, bm = tm;
+    }
+  }
+  return splits;
+}
+
+// The rule of the 4-bit form, whose single passes go through registers and stand further behind: flops at 900 (128 x 128) or 700 (64 x 128) TFLOP/s
+// times how full the last round of 512 workgroups is, and the partials there and back at 9 TB/s (they stay in the last-level cache).  Measured, us
+// (without | chosen here | by the rule above): 512 x 2048 x 8192 88 | 48 | 88; 1486 x 1280 x 5120 79 | 45 | 79; 2048 x 1536 x 8960 143 | 100 | 107;
+// 386 x 4096 x 4096 62 | 38 | 62; 165 products together 0.805 of their time without, by the rule above 0.834; the worst 27.8 | 29.0.
+int wide_split_w4(int M, int N, int K, int& bm) {
   const long t128 = (long)vlm_cdiv(M, 128) * vlm_cdiv(N, 128);
   if (M <= 64 || K < 4096 || t128 >= 512 || (t128 > 256 && K < 16384)) return 0;
   const auto fill = [](long wgs) { return (double)wgs / (512. * ((wgs + 511) / 512)); };
@@ -824,11 +859,11 @@ int launch_epi_w4(const void* A, const void* Wq, const void* Wsb, const void* bi
                   int lda, int ldc, int ldres, hipStream_t st) {
   const long t128 = (long)vlm_cdiv(M, 128) * vlm_cdiv(N, 128);
   const long t64n = (long)vlm_cdiv(M, 64) * vlm_cdiv(N, 128);
-  if (!(EPI & VLM_EPI_SWIGLU) && g_splitk >= 0 && N % 8 == 0) {          // same split-K policy as the bf16 form
+  if (!(EPI & VLM_EPI_SWIGLU) && g_splitk >= 0 && N % 8 == 0) {          // (split as the bf16 form is but for the wide tiles' own rule)
     const long t64 = (long)vlm_cdiv(M, 64) * vlm_cdiv(N, 64);
     int splits = g_splitk > 1 ? g_splitk : 0, bm = 0;
     if (!splits && K % BK == 0)
-      if (const int wide = wide_split(M, N, K, bm))
+      if (const int wide = wide_split_w4(M, N, K, bm))
         if (float* ws = splitk_workspace((size_t)wide * M * N * sizeof(float), st))
           return bm == 128 ? launch_splitk_w4<EPI, 128, 128>(A, Wq, Wsb, bias, res, C, M, N, K, lda, ldc, ldres, wide, ws, st)
                            : launch_splitk_w4<EPI, 64, 128>(A, Wq, Wsb, bias, res, C, M, N, K, lda, ldc, ldres, wide, ws, st);

@@ -968,6 +968,20 @@ def test_gemm_wide_tiles_split_and_staged(vops, M, N, K, epi):
     assert torch.equal(vops.gemm(a, w, **kw), got)
 
 
+@pytest.mark.parametrize("M,N,K,split", [(386, 4096, 4096, False), (512, 4096, 4096, False), (2048, 1024, 4096, False), (386, 3072, 8192, True), (1020, 1280, 5120, True)])
+def test_long_products_are_split_only_where_it_pays(vops, M, N, K, split):
+    """a product that one pass of 64 x 64 tiles does sooner keeps to one sum over K (the bits of the pass that is never split), one that leaves
+    compute units idle is split"""
+    a, w = rnd(M, K, seed=M).cuda(), rnd(N, K, seed=N, scale=0.3).cuda()
+    got = vops.gemm(a, w)
+    vops.gemm_set_staging(8)
+    try:
+        whole = vops.gemm(a, w)
+    finally:
+        vops.gemm_set_staging(0)
+    assert torch.equal(got, whole) is (not split)
+
+
 @pytest.mark.parametrize("M,H,hd", [(9216, 16, 80), (1024, 16, 80), (200, 2, 80), (77, 3, 64)])
 def test_gemm_rope2d_epilogue_equals_gemm_then_rope_pass(vops, M, H, hd):
     """vlm_gemm_bf16_rope2d (2-D rope of the vision attention in the qkv GEMM epilogue, q / k rows interleaved per head)
