@@ -169,13 +169,13 @@ class LanguageModel(RaggedLanguageModel):
             ops.headnorm_rows(col("k"), G, D, pl.tok_pos, kpool, eps=eps, raw_dim=Dv, **rot, **paged)
             ops.headnorm_rows(col("q"), H, D, pl.tok_pos, q, eps=eps, **rot)
         out = torch.empty(Tn, _al8(H * Dv), dtype=self.dtype, device=dev)[:, : H * Dv]
-        # prompt form wherever a step brings more than decode rows, and always in float32 serving - one kernel there, so that
+        # prompt form wherever a step brings more than decode rows or few keys (_few_keys), and always in float32 serving - one kernel there, so that
         # a token's bits do not depend on the schedule (shapes its LDS tiles cannot take run the row form everywhere)
         DP = (D + 3) & ~3
         nacc = 4 if Dv <= 64 else (8 if Dv <= 128 else 16)
         blocks_fit = Dv <= 256 and (16 * DP + 16 * (DP + 4) + 16 * nacc * 16 + 16 * 17 + 48) * 4 <= 48 * 1024
         args = dict(window=ns.window, gate=col("g"), sink=not whole_row_norm)
-        if (self.dtype == torch.float32 or Tn > 8) and blocks_fit:
+        if (self.dtype == torch.float32 or Tn > 8 and not self._few_keys(pl, ns.window)) and blocks_fit:
             ops.window_attn_blocks(q, kpool, vpool, pl.qb_start, pl.qb_count, pl.tok_seq, pl.tok_pos, pool.block_table, H, G, D, Dv,
                                    ns.scale, out, **args)
         else:

@@ -204,9 +204,9 @@ class LanguageModel(RaggedLanguageModel):
                                stride_c=R + Dr)
                 if Dr:
                     ops.rope_pairs_rows(proj[:, ns.off["q"] + D:], D + Dr, H, Dr, ns.inv_freq, tok_pos_d, qabs[:, R:], R + Dr)
-                # prompt form (key tiles shared by a block of queries) wherever a step brings more than decode rows, and always
+                # prompt form (key tiles shared by a block of queries) wherever a step brings more than decode rows or few keys (_few_keys), and always
                 # in float32 serving - one kernel there, so that a token's bits do not depend on the schedule
-                if (is32 or Tn > 8) and R <= 512 and (32 * _al8(R + Dr) + 512) * 4 <= 150 * 1024:
+                if (is32 or Tn > 8 and not self._few_keys(pl)) and R <= 512 and (32 * _al8(R + Dr) + 512) * 4 <= 150 * 1024:
                     ol = ops.latent_attn_blocks(qabs.view(Tn, H, R + Dr), pool.rows[ns.src], pl.qb_start, pl.qb_count, tok_seq_d, tok_pos_d,
                                                 bt, H, R, Dr, ns.scale, gate=col("g"))
                 else:

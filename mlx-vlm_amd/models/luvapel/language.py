@@ -196,9 +196,9 @@ class LanguageModel(RaggedLanguageModel):
         q = torch.empty(Tn, H * D, dtype=torch.float32, device=dev)
         ops.headnorm_rope_rows(col("lq"), H, D, ns.qnorm, eps, ns.rot_dims, ns.inv_freq, pl.tok_pos, q)
         out = torch.empty(Tn, H * D, dtype=self.dtype, device=dev)
-        # prompt form wherever a step brings more than decode rows, and always in float32 serving - one kernel there, so that
+        # prompt form wherever a step brings more than decode rows or few keys (_few_keys), and always in float32 serving - one kernel there, so that
         # a token's bits do not depend on the schedule
-        if self.dtype == torch.float32 or Tn > 8:
+        if self.dtype == torch.float32 or Tn > 8 and not self._few_keys(pl, ns.window):
             ops.window_attn_blocks(q, kpool, vpool, pl.qb_start, pl.qb_count, pl.tok_seq, pl.tok_pos, pool.block_table, H, G, D, D,
                                    ns.scale, out, temp=ns.temp, window=ns.window, gate=col("lg"))
         else:

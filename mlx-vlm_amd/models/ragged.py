@@ -234,13 +234,21 @@ class RaggedLanguageModel:
                                .reshape(-1).to(torch.int32) for _, ids in entries])
         return SimpleNamespace(seqs=seqs, lens=lens, nseg=nseg, Tn=Tn, rows=rows, all_rows=bool(rows.size == Tn and np.array_equal(rows, np.arange(Tn))),
                                tok_seq=parts[0], tok_pos=parts[1], cu=parts[2], slot=parts[3], pos0=parts[4], rows_d=parts[5], qb_start=parts[6],
-                               qb_count=parts[7], ids=ids_d, md=md, keys=self._keys(seqs))
+                               qb_count=parts[7], ids=ids_d, md=md, keys=self._keys(seqs) if Tn == nseg else max(s.offset + n for s, n in zip(seqs, lens)))
 
     @staticmethod
     def _keys(seqs):
         """the most tokens that the pages reserved for any of these sequences hold: generation reserves what a request may grow to before
         its first step, so that this says, steadily over its steps, how long its context can get"""
         return max(len(s.pages) for s in seqs) * PAGE
+
+    def _few_keys(self, pl, window=0):
+        """whether the tokens of a prompt step are few and see few keys: bf16 prompts of up to 160 tokens over up to 64 keys take the scalar
+        row kernels of attention.  us, scalar blocks of 16 queries | blocks on the matrix cores | rows: windowed, 12 heads (2) of 128, 16
+        tokens 8.5 | 17.5 | 5.5, 8 x 20 12.8 | 17.8 | 9.0, 2 x 64 22 | 18.0 | 9.3; 28 heads (4), 8 x 20 14.4 | 17.9 | 15.6, 3 x 53 25 | 18.1 | 17.4;
+        latent R = 512, 12 heads, 16 tokens 16.5 | 22.5 | 7.2, 2 x 64 38 | 23.4 | 13.6; 28 heads, 2 x 64 39 | 24.0 | 24.7.  (256 tokens, windowed, 16 heads
+        of 96: 11.7 | 11.4 | 14.6.)  Decode rows are never taken: their step may be captured, and a graph is kept for any context."""
+        return self.dtype == torch.bfloat16 and pl.nseg < pl.Tn <= 160 and min(pl.keys, window or pl.keys) <= 64
 
     _trace = None      # a list: step() appends the stream after every layer (debugging / tests)
 

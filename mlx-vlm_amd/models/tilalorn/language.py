@@ -133,13 +133,13 @@ class LanguageModel(RaggedLanguageModel):
         q = torch.empty(Tn, H * D, dtype=torch.float32, device=dev)
         ops.headnorm_rows(col("q"), H, D, pl.tok_pos, q, eps=eps, bias=ns.qb, temp=ns.q_temp)
         out = torch.empty(Tn, _al8(H * Dv), dtype=self.dtype, device=dev)[:, : H * Dv]
-        # prompt form wherever a step brings more than decode rows, and always in float32 serving - one kernel there, so that
+        # prompt form wherever a step brings more than decode rows or few keys (_few_keys), and always in float32 serving - one kernel there, so that
         # a token's bits do not depend on the schedule (shapes its LDS tiles cannot take run the row form everywhere)
         DP = (D + 3) & ~3
         nacc = 4 if Dv <= 64 else (8 if Dv <= 128 else 16)
         blocks_fit = Dv <= 256 and (16 * DP + 16 * (DP + 4) + 16 * nacc * 16 + 16 * 17 + 48) * 4 <= 48 * 1024
         args = dict(temp=None, window=ns.window, gate=col("g"), cap=ns.cap, gate_head=True)
-        if (self.dtype == torch.float32 or Tn > 8) and blocks_fit:
+        if (self.dtype == torch.float32 or Tn > 8 and not self._few_keys(pl, ns.window)) and blocks_fit:
             ops.window_attn_blocks(q, kpool, vpool, pl.qb_start, pl.qb_count, pl.tok_seq, pl.tok_pos, pool.block_table, H, G, D, Dv,
                                    ns.scale, out, **args)
         else:
@@ -162,7 +162,7 @@ class LanguageModel(RaggedLanguageModel):
         ops.linear_any(col("q"), ns.uk_t.view(H * R, D), out=qabs, M=Tn, N=R, K=D, batch=H, stride_a=D + Dr, stride_w=R * D, stride_c=R + Dr)
         if Dr:
             ops.rope_pairs_rows(proj[:, ns.off["q"] + D:], D + Dr, H, Dr, ns.inv_freq, pl.tok_pos, qabs[:, R:], R + Dr, rot_half=True)
-        if (self.dtype == torch.float32 or Tn > 8) and R <= 512 and (32 * _al8(R + Dr) + 512) * 4 <= 150 * 1024:
+        if (self.dtype == torch.float32 or Tn > 8 and not self._few_keys(pl, ns.window)) and R <= 512 and (32 * _al8(R + Dr) + 512) * 4 <= 150 * 1024:
             ol = ops.latent_attn_blocks(qabs.view(Tn, H, R + Dr), cpool, pl.qb_start, pl.qb_count, pl.tok_seq, pl.tok_pos, bt, H, R, Dr,
                                         ns.scale, window=ns.window)
         else:

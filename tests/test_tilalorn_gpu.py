@@ -782,6 +782,27 @@ def test_decode_rows_of_short_contexts_take_the_scalar_kernels(tmp_path, monkeyp
     assert H.rel_rms(torch.stack([l for l, _ in eager[1:]]), want) < TOL["bfloat16"]
 
 
+@pytest.mark.parametrize("lens,held,rows", [([64], 0, True), ([65], 0, False), ([32] * 5, 0, True), ([32] * 4 + [33], 0, False), ([60, 5], 0, True), ([20], 44, True), ([20], 45, False)])
+def test_prompts_of_few_tokens_over_few_keys_take_the_row_kernels(tmp_path, monkeypatch, lens, held, rows):
+    """both sides of the lines (160 tokens of a step, 64 keys of a token): which kernels run, and the logits against float64"""
+    from mlx_vlm_amd import ops
+
+    cfg = H.config([H.latent(kv_rank=136, window=0, mlp="dense"), H.attention(window=0)])
+    W = H.weights(cfg, seed=4)
+    lm = _load(tmp_path, cfg, W, "bfloat16", tokens=4096, seqs=8).language_model
+    texts = [_ids(held + n, cfg["vocab"], 30 + i) for i, n in enumerate(lens)]
+    caches = [lm.make_cache() for _ in texts]
+    if held:
+        lm.step([(c[0]._seq, t[:held]) for c, t in zip(caches, texts)])
+    calls = []
+    for name in ("latent_attn", "latent_attn_blocks", "window_attn_rows", "window_attn_blocks"):
+        monkeypatch.setattr(ops, name, lambda *a, name=name, real=getattr(ops, name), **kw: (calls.append(name), real(*a, **kw))[1])
+    got = lm.step([(c[0]._seq, t[held:]) for c, t in zip(caches, texts)], want="all").cpu()
+    assert calls == (["latent_attn", "window_attn_rows"] if rows else ["latent_attn_blocks", "window_attn_blocks"])
+    orc = O.Oracle(cfg, W, F64)
+    assert H.rel_rms(got, torch.cat([orc.forward(t)[held:] for t in texts])) < TOL["bfloat16"]
+
+
 def test_sampled_generation_uses_the_device_sampler_and_refuses_what_is_not_built(tmp_path):
     from mlx_vlm_amd.generate import generate_step
 
