@@ -16,8 +16,8 @@
 //                            first, an RMS norm WITHOUT a weight, a multiplier that grows with the logarithm of the position
 //                            (1 + coef * ln(floor((pos + 1) / every) + 1), for queries), and separately projected value rows
 //                            [T][heads][Dv] (+ bias) copied into their own paged pool in the same launch.
-//   vlm_window_attn_blocks   prompt form (fp32 values; bf16 values run on the matrix cores: grouped_attn.hip): workgroup = (block of up to 16 consecutive queries of one sequence, head); tiles of 16
-//                            keys at multiples of 16 counted from the sequence's first token go through LDS once per block, and
+//   vlm_window_attn_blocks   prompt form (fp32 values, and bf16 values under windows of up to 16; else those run on the matrix cores:
+//                            grouped_attn.hip): workgroup = (block of up to 16 consecutive queries of one sequence, head); tiles of 16 keys at multiples of 16 counted from the sequence's first token go through LDS once per block, and
 //                            every query runs the same per-tile update in the same order whatever block it sits in (a tile with
 //                            no visible key leaves its running maximum, sum and accumulator untouched bit for bit): a token's
 //                            result does not depend on how the prompt was cut or batched.
@@ -480,7 +480,10 @@ extern "C" int vlm_window_attn_blocks(const void* q, const void* kpool, const vo
   const int DP = (D + 3) & ~3;
   const size_t lds = ((size_t)QB * DP + (size_t)KT * (DP + 4) + (size_t)KT * nacc * 16 + QB * (KT + 1) + 3 * QB) * sizeof(float);
   if (Dv > 256 || H > 65535 || lds > 48 * 1024) return VLM_ERR_SHAPE;
-  if (!dtype) {                                          // bf16 values: the matrix cores (fp32: one summation order whatever the schedule)
+  // bf16 values: the matrix cores (fp32: one summation order whatever the schedule), but for windows that two tiles of 16 keys hold, us here |
+  // there: 12 heads (2) of 128, window 16, 256 tokens 13.0 | 18.0, 4096 59 | 68; 28 heads (4), 4096 130 | 170; 16 heads of 96, 1024 17.5 | 22.8;
+  // 4 heads of 64, 256 9.9 | 7.9.  Window 32: 17.7 | 18.2, 81 | 68; 179 | 170; 26.9 | 23.1; 13.0 | 8.0.
+  if (!dtype && !(window > 0 && window <= 16)) {
     vlm_grouped_attn_args a = {};
     a.q = (const float*)q; a.kpool = kpool; a.vpool = vpool; a.qb_start = (const int*)qb_start; a.qb_count = (const int*)qb_count;
     a.tok_seq = (const int*)tok_seq; a.tok_pos = (const int*)tok_pos; a.block_table = (const int*)block_table;
@@ -490,11 +493,15 @@ extern "C" int vlm_window_attn_blocks(const void* q, const void* kpool, const vo
   }
   hipStream_t st = (hipStream_t)stream;
   dim3 grid(nblocks, H);
-#define GO(N)                                                                                                                       \
-  hipLaunchKernelGGL((window_attn_block_kernel<float, N>), grid, dim3(256), lds, st, (const float*)q, (const float*)kpool, (const float*)vpool, \
+#define GO(T, N)                                                                                                                    \
+  hipLaunchKernelGGL((window_attn_block_kernel<T, N>), grid, dim3(256), lds, st, (const float*)q, (const float*)kpool, (const T*)vpool, \
                      (const int*)qb_start, (const int*)qb_count, (const int*)tok_seq, (const int*)tok_pos, (const int*)block_table,  \
-                     max_pages, H, KH, D, Dv, scale, (const float*)temp, window, cap, sink, (const float*)gate, ldgate, gate_head, (float*)out, ldo)
-  if (nacc == 4) GO(4); else if (nacc == 8) GO(8); else GO(16);
+                     max_pages, H, KH, D, Dv, scale, (const T*)temp, window, cap, sink, (const T*)gate, ldgate, gate_head, (T*)out, ldo)
+  if (dtype) {
+    if (nacc == 4) GO(float, 4); else if (nacc == 8) GO(float, 8); else GO(float, 16);
+  } else {
+    if (nacc == 4) GO(bf16_t, 4); else if (nacc == 8) GO(bf16_t, 8); else GO(bf16_t, 16);
+  }
 #undef GO
   VLM_CHECK_LAUNCH();
   return VLM_OK;

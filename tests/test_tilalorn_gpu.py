@@ -289,6 +289,28 @@ def test_window_attention_f32_keys_over_bf16_values(D, Dv, Hh, KH):
             assert bool(((out.double().view(T, Hh, Dv) - want).abs() <= bound).all()), (form.__name__, window, cap)
 
 
+@pytest.mark.parametrize("window,same", [(1, True), (15, True), (16, True), (17, False)])
+@pytest.mark.parametrize("D,Dv,Hh,KH", [(128, 128, 12, 2), (96, 96, 5, 5), (30, 17, 3, 3)])
+def test_windows_of_a_few_keys_are_read_by_the_scalar_blocks(D, Dv, Hh, KH, window, same):
+    """up to a window of 16 bf16 values are summed as fp32 ones are, in tiles of 16 keys: the same bits but for the rounding of the output; from 17 on
+    on the matrix cores, sums in another order"""
+    from mlx_vlm_amd import ops
+    from mlx_vlm_amd.models.cache import PAGE
+
+    g = torch.Generator().manual_seed(window)
+    T, npg = 200, 4
+    q, kpool, vpool = torch.randn(T, Hh * D, generator=g).cuda(), torch.randn(npg, PAGE, KH * D, generator=g).cuda(), torch.randn(npg, PAGE, KH * Dv, generator=g).bfloat16().cuda()
+    qs = torch.arange(0, T, 16, dtype=torch.int32).cuda()
+    args = (qs, (T - qs).clamp(max=16), torch.zeros(T, dtype=torch.int32).cuda(), torch.arange(T, dtype=torch.int32).cuda(), torch.arange(npg, dtype=torch.int32).view(1, npg).cuda(),
+            Hh, KH, D, Dv, 2 * D ** -0.5)
+    got, want = torch.empty(T, Hh * Dv, dtype=torch.bfloat16, device="cuda"), torch.empty(T, Hh * Dv, device="cuda")
+    ops.window_attn_blocks(q, kpool, vpool, *args, got, window=window, cap=9.0)
+    ops.window_attn_blocks(q, kpool, vpool.float(), *args, want, window=window, cap=9.0)
+    if same:
+        assert torch.equal(got, want.bfloat16())
+    assert bool(((got.float() - want).abs() <= want.abs() * 2.0 ** -8 + 2 ** -23 * 2 * (D + 16) / 100 * float(want.abs().max())).all())
+
+
 @pytest.mark.parametrize("R,Dr,Hh", [(512, 64, 5), (512, 0, 4), (136, 24, 9), (256, 64, 17), (128, 64, 16), (8, 0, 1)])
 def test_latent_attention_f32_queries_over_bf16_rows(R, Dr, Hh):
     """the matrix-core forms take all 24 bits of a query and of a weight: as near to float64 as sums of fp32 are (a score is a sum of R + Dr
