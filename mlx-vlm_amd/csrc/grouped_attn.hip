@@ -237,7 +237,8 @@ __global__ __launch_bounds__(NW * 64) void grouped_attn_kernel(vlm_grouped_attn_
   const int pos0 = p.tok_pos[t0], last = decode ? pos0 : pos0 + ncol - 1;
   const int window = p.window;
   const int tiles = last / KTL + 1;
-  const int first_tile = window > 0 ? max(0, pos0 - window + 1) / KTL : 0;   // holds the first query's oldest visible key
+  const int oldest = window > 0 ? max(0, pos0 - window + 1) : 0;             // the first query's oldest visible key
+  const int first_tile = oldest / KTL;
   const bool split = gridDim.z > 1;
   if (split && first_tile + (int)blockIdx.z * NW >= tiles) {              // no keys for this workgroup: only the marks of an empty part (uniform)
     if (tid < ncol) {
@@ -291,7 +292,10 @@ __global__ __launch_bounds__(NW * 64) void grouped_attn_kernel(vlm_grouped_attn_
   const int nw = NW * gridDim.z;
   for (int j = first_tile + blockIdx.z * NW + wave; j < tiles; j += nw) {
     const long prow = (long)bt[j / (PAGE / KTL)] * PAGE + (j % (PAGE / KTL)) * KTL;
-    const int lim = last - j * KTL;                                       // place of the last key that exists (may be past the tile)
+    // places of the oldest and the last key that is seen (may be before and past the tile): the others' rows are not read, as a zero weight
+    // would hand on what is not finite there
+    const int from = oldest - j * KTL, lim = last - j * KTL;
+    const auto place = [&](int key) { return max(min(key, lim), from); };
     f32x4_t s[U][CG];
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -299,7 +303,7 @@ __global__ __launch_bounds__(NW * 64) void grouped_attn_kernel(vlm_grouped_attn_
       for (int m = 0; m < CG; ++m) s[u][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     bool done = false;
     if constexpr (MIX && NB <= 8) {
-      const TK *k0 = kbase + (prow + min(r16, lim)) * krow_sz, *k1 = kbase + (prow + min(16 + r16, lim)) * krow_sz;
+      const TK *k0 = kbase + (prow + place(r16)) * krow_sz, *k1 = kbase + (prow + place(16 + r16)) * krow_sz;
       if (D == 128) scores32<CG, 8>(k0, k1, qs, QP, r16, g, s);
       else if (D == 64) scores32<CG, 4>(k0, k1, qs, QP, r16, g, s);
       done = D == 128 || D == 64;
@@ -307,7 +311,7 @@ __global__ __launch_bounds__(NW * 64) void grouped_attn_kernel(vlm_grouped_attn_
     if (!done)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const TK* kr = kbase + (prow + min(16 * u + r16, lim)) * krow_sz;
+      const TK* kr = kbase + (prow + place(16 * u + r16)) * krow_sz;
       if constexpr (F32) scores16<CG>(kr, dvec, D, DP, qs, QP, r16, g, s[u]);
       else scores16<CG>(kr, D8, qb, QPB, r16, g, s[u]);
     }
@@ -316,7 +320,7 @@ __global__ __launch_bounds__(NW * 64) void grouped_attn_kernel(vlm_grouped_attn_
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[u * 4 + r].load(vbase + (prow + min(16 * u + 4 * g + r, lim)) * vrow_sz, vhave, vvec);
+      for (int r = 0; r < 4; ++r) v[u * 4 + r].load(vbase + (prow + place(16 * u + 4 * g + r)) * vrow_sz, vhave, vvec);
     // a tile that every query of the workgroup sees in full needs no mask
     const int tile_lo = j * KTL, tile_hi = tile_lo + KTL - 1;
     const bool full = tile_hi <= pos0 && (window <= 0 || last - tile_lo < window);

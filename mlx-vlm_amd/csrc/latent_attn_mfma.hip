@@ -94,7 +94,8 @@ template <int NKS> __device__ __forceinline__ void load_queries(const float* qro
 }
 
 // copies of a page's rows into a tile by 256 threads: this thread's pieces are tid, tid + 256, ... (a page's rows are contiguous in memory);
-// rows past the last key repeat its last piece (they are masked)
+// rows past the last key repeat its last piece (they are masked); the first `skip` rows of a page, which no query sees, are zeros: a zero weight
+// would hand on what is not finite there
 template <int NKS> struct Stager {
   static constexpr int PARTS = NKS % 3 == 0 ? 3 : 2, HALF = NKS / PARTS;          // a page goes through the registers in parts
   int loff[NKS], pieces, D8;
@@ -113,11 +114,15 @@ template <int NKS> struct Stager {
       *reinterpret_cast<u32x4_t*>(tiles + (i / (pad * PAGE)) * Tile<NKS>::SIZE + row * Tile<NKS>::PITCH + (D8 + i % pad) * 8) = u32x4_t{0u, 0u, 0u, 0u};
     }
   }
-  template <int H> __device__ __forceinline__ void load(const bf16_t* page, int keys, int tid) {
+  template <int H> __device__ __forceinline__ void load(const bf16_t* page, int keys, int tid, int skip = 0) {
     const u32x4_t* src = reinterpret_cast<const u32x4_t*>(page);
     const int have = min(pieces, keys * D8) - 1;
 #pragma unroll
     for (int i = 0; i < HALF; ++i) st[i] = src[min(tid + 256 * (H * HALF + i), have)];
+    if (skip > 0)
+#pragma unroll
+      for (int i = 0; i < HALF; ++i)
+        if (tid + 256 * (H * HALF + i) < skip * D8) st[i] = u32x4_t{0u, 0u, 0u, 0u};
   }
   template <int H> __device__ __forceinline__ void store(bf16_t* tile) {
 #pragma unroll
@@ -202,10 +207,10 @@ __global__ __launch_bounds__(256, 1) void latent_block_mfma_kernel(vlm_latent_mf
   const int pos0 = p.tok_pos[t0], last = pos0 + nq - 1, mypos = r16 < nq ? pos0 + r16 : -1, window = p.window;
   const float sc = p.scale * LOG2E;
   const bf16_t* pool = (const bf16_t*)p.pool;
-  const int first = window > 0 ? max(0, pos0 - window + 1) / PAGE : 0, tiles = last / PAGE + 1;
+  const int oldest = window > 0 ? max(0, pos0 - window + 1) : 0, first = oldest / PAGE, tiles = last / PAGE + 1;
   Stager<NKS> sg;
   sg.init(tile, 2, Dk, tid);
-  sg.template load<0>(pool + (long)bt[first] * PAGE * Dk, last - first * PAGE + 1, tid);
+  sg.template load<0>(pool + (long)bt[first] * PAGE * Dk, last - first * PAGE + 1, tid, oldest % PAGE);
   bf8 q[NKS][NQ<TQ>];
   load_queries<NKS>((const TQ*)p.q + ((long)(t0 + r16) * p.H + h) * Dk, live && r16 < nq, Dk, g, q);
   f32x4_t acc[NVC][8];
@@ -215,10 +220,10 @@ __global__ __launch_bounds__(256, 1) void latent_block_mfma_kernel(vlm_latent_mf
     for (int b = 0; b < 8; ++b) acc[c][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float mrun = -INFINITY, lrun = 0.f;
   sg.template store<0>(tile);
-  sg.template load<1>(pool + (long)bt[first] * PAGE * Dk, last - first * PAGE + 1, tid);
+  sg.template load<1>(pool + (long)bt[first] * PAGE * Dk, last - first * PAGE + 1, tid, oldest % PAGE);
   sg.template store<1>(tile);
   if constexpr (Stager<NKS>::PARTS > 2) {
-    sg.template load<2>(pool + (long)bt[first] * PAGE * Dk, last - first * PAGE + 1, tid);
+    sg.template load<2>(pool + (long)bt[first] * PAGE * Dk, last - first * PAGE + 1, tid, oldest % PAGE);
     sg.template store<2>(tile);
   }
   for (int j = first; j < tiles; ++j) {
@@ -316,7 +321,7 @@ __global__ __launch_bounds__(256) void latent_rows_mfma_kernel(vlm_latent_mfma_a
   const int t = blockIdx.x, h0 = blockIdx.y * QC, ncol = min(QC, p.H - h0), z = blockIdx.z;
   const int* bt = p.block_table + (long)p.tok_seq[t] * p.max_pages;
   const int pos = p.tok_pos[t], window = p.window;
-  const int first = window > 0 ? max(0, pos - window + 1) / PAGE : 0, tiles = pos / PAGE + 1;
+  const int oldest = window > 0 ? max(0, pos - window + 1) : 0, first = oldest / PAGE, tiles = pos / PAGE + 1;
   const bool split = gridDim.z > 1;
   const float sc = p.scale * LOG2E;
   float* part = p.part + (((long)z * p.H + h0 + r16) * gridDim.x + t) * (R + 2);        // of this lane's column
@@ -340,9 +345,13 @@ __global__ __launch_bounds__(256) void latent_rows_mfma_kernel(vlm_latent_mfma_a
     const bf16_t* page = pool + (long)bt[j] * PAGE * Dk;
     u32x4_t st[NKS];                                     // (the whole page in flight at once)
     const u32x4_t* src = reinterpret_cast<const u32x4_t*>(page);
-    const int have = min(sg.pieces, (pos - j * PAGE + 1) * sg.D8) - 1;
+    const int skip = (oldest - j * PAGE) * sg.D8, have = min(sg.pieces, (pos - j * PAGE + 1) * sg.D8) - 1;
 #pragma unroll
     for (int i = 0; i < NKS; ++i) st[i] = src[min(tid + 256 * i, have)];
+    if (skip > 0)
+#pragma unroll
+      for (int i = 0; i < NKS; ++i)
+        if (tid + 256 * i < skip) st[i] = u32x4_t{0u, 0u, 0u, 0u};
     __syncthreads();                                     // (everybody is through with the previous page and its scores)
 #pragma unroll
     for (int i = 0; i < NKS; ++i) *reinterpret_cast<u32x4_t*>(tile + sg.loff[i]) = st[i];

@@ -311,6 +311,41 @@ def test_windows_of_a_few_keys_are_read_by_the_scalar_blocks(D, Dv, Hh, KH, wind
     assert bool(((got.float() - want).abs() <= want.abs() * 2.0 ** -8 + 2 ** -23 * 2 * (D + 16) / 100 * float(want.abs().max())).all())
 
 
+@pytest.mark.parametrize("form", ["rows", "blocks"])
+@pytest.mark.parametrize("kind,sizes", [("windowed", (128, 128)), ("windowed", (96, 40)), ("windowed", (160, 256)), ("latent", (512, 64)), ("latent", (128, 32))])
+def test_keys_before_every_window_are_not_read(kind, sizes, form):
+    """values that are not finite in the rows before the oldest key that a query sees leave its read-out as it is, also where the matrix cores take
+    that key's tile or page from its beginning"""
+    from mlx_vlm_amd import ops
+    from mlx_vlm_amd.models.cache import PAGE
+
+    g = torch.Generator().manual_seed(sizes[0])
+    npg, (a, b) = 3, sizes
+    for pos, n, window in ((127, 1, 40), (120, 16, 57), (150, 3, 65), (191, 1, 17)):          # (first query's position, queries)
+        n = 1 if form == "rows" else n
+        oldest, D, W = pos - window + 1, a if kind == "windowed" else a + b, b if kind == "windowed" else a
+        q = torch.randn(n, 4 * D, generator=g).cuda()
+        kpool = torch.randn(npg, PAGE, 2 * D if kind == "windowed" else D, generator=g).cuda()
+        vpool = torch.randn(npg, PAGE, 2 * b, generator=g).bfloat16().cuda()
+        bt = torch.randperm(npg, generator=g).to(torch.int32).view(1, npg).cuda()
+        at = (torch.zeros(n, dtype=torch.int32).cuda(), torch.arange(pos, pos + n, dtype=torch.int32).cuda(), bt)
+        blk = (torch.tensor([0], dtype=torch.int32).cuda(), torch.tensor([n], dtype=torch.int32).cuda()) if form == "blocks" else ()
+        got = []
+        for bad in (None, float("nan"), float("inf")):
+            k, v = kpool.clone() if kind == "windowed" else kpool.bfloat16(), vpool.clone()
+            if bad is not None:
+                for i in range(oldest):
+                    k[int(bt[0, i // PAGE]), i % PAGE] = bad
+                    v[int(bt[0, i // PAGE]), i % PAGE] = bad
+            if kind == "windowed":
+                out = torch.empty(n, 4 * W, dtype=torch.bfloat16, device="cuda")
+                getattr(ops, "window_attn_" + form)(q, k, v, *blk, *at, 4, 2, D, W, D ** -0.5, out, window=window)
+            else:
+                out = (ops.latent_attn_blocks if blk else ops.latent_attn)(q.view(n, 4, D), k, *blk, *at, 4, a, b, D ** -0.5, window=window)
+            got.append(out)
+        assert bool(got[0].isfinite().all()) and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2]), (pos, n, window)
+
+
 @pytest.mark.parametrize("R,Dr,Hh", [(512, 64, 5), (512, 0, 4), (136, 24, 9), (256, 64, 17), (128, 64, 16), (8, 0, 1)])
 def test_latent_attention_f32_queries_over_bf16_rows(R, Dr, Hh):
     """the matrix-core forms take all 24 bits of a query and of a weight: as near to float64 as sums of fp32 are (a score is a sum of R + Dr
