@@ -160,10 +160,12 @@ class RaggedLanguageModel:
         if mfma and accumulate and K > 4096 and N <= 8192 and (3 <= M <= 8 or (M == 2 and K > 20480)) and skip is None:
             return ops.linear_any(a, w, out=out, out_dtype=out_dtype, accumulate=accumulate)
         # a long K is split over workgroups, in a capture too ([1536, 17920], 2 / 3 / 4 / 8 rows: 17 / 17 / 17 / 17; streaming 22 / 64 / 72 / 114, and over the zeros
-        # of unchosen experts 20 / 47 / 58 / 100; one pass 66).  Two rows from K = 8192 and below 16384 columns ([1536, 4736] 9.9, streaming 7.9; [1536, 6720] 10.5 and
-        # 10.0; [1536, 8960] 11.7 and 12.2; [35840, 4608] 70 and 56); three on a par at [4608, 4608] (15.5 and 15.1).  With `skip` up to STREAM_ROWS rows
+        # of unchosen experts 20 / 47 / 58 / 100; one pass 66); three rows on a par at [4608, 4608] (15.5 and 15.1) and [8192, 8192] (34.8 and 35.3).  Two rows stay
+        # with the streaming form while four of its workgroups fit a compute unit (40 KB of activations each) or columns fill the chip, split | streaming:
+        # [1536, 8960] 12.5 | 12.7 in two launches, [3584, 9472] 18.8 | 19.6, [4608, 8960] 23 | 20, [8192, 8192] 35 | 27, [12288, 12288] 77 | 58, [7168, 20480] 76 | 62;
+        # [2560, 16384] 27 | 36, [4096, 11008] 24 | 35, [5120, 13824] 36 | 40, [6144, 16384] 48 | 50.  With `skip` up to STREAM_ROWS rows
         # stay with the form that leaves columns out ([35840, 4608], two of eight experts a row, 2 / 3 / 4 rows 37 / 50 / 69, the GEMM 70 / 69 / 70)
-        split = K > 4096 and K % 64 == 0 and skip is None and (M > 2 or (M == 2 and K >= 8192 and N < 16384))
+        split = K > 4096 and K % 64 == 0 and skip is None and (M > 2 or (M == 2 and (K > 20480 and N < 16384 or K > 10240 and N <= 6144)))
         if (mfma and not accumulate and want == torch.bfloat16 and (M > self.STREAM_ROWS or split) and N % 8 == 0
                 and (out is None or (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0))):
             return ops.gemm_rows(a, w, out=out) if M <= 64 and K > 4096 else ops.gemm(a, w, out=out)

@@ -139,7 +139,8 @@ def test_oracle_router_keeps_the_best_groups_and_does_not_renormalise():
 @pytest.mark.parametrize("M,N,K,skip,route", [
     (2, 4096, 4608, True, "linear_rows_bf16w"), (3, 4096, 4608, True, "linear_rows_bf16w"), (4, 4096, 4608, True, "linear_rows_bf16w"),      # the columns of experts are left out
     (5, 4096, 4608, False, "gemm_rows"), (4, 4096, 4608, False, "gemm_rows"), (3, 4096, 4616, False, "linear_rows_bf16w"),             # (a K that is not split)
-    (2, 1536, 4736, False, "linear_rows_bf16w"), (2, 1536, 8960, False, "gemm_rows"), (2, 16384, 8960, False, "linear_rows_bf16w"), (1, 1536, 17920, False, "linear_rows_bf16w"),
+    (2, 1536, 4736, False, "linear_rows_bf16w"), (2, 1536, 8960, False, "linear_rows_bf16w"), (2, 1536, 17920, False, "gemm_rows"), (2, 6144, 10304, False, "gemm_rows"),
+    (2, 8192, 16384, False, "linear_rows_bf16w"), (2, 8192, 20544, False, "gemm_rows"), (2, 16384, 20544, False, "linear_rows_bf16w"), (1, 1536, 17920, False, "linear_rows_bf16w"),
     (3, 1536, 1536, False, "linear_any"), (3, 1536, 1536, True, "linear_rows_bf16w"), (65, 1536, 4608, False, "gemm")])
 def test_products_of_few_rows_take_the_form_that_was_measured_for_them(monkeypatch, M, N, K, skip, route):
     """up to STREAM_ROWS rows with an expert table keep the form that leaves columns out, whatever K"""
