@@ -302,6 +302,38 @@ def test_a_workspace_changes_no_recurrence(gated, rot, q_act, decays):
         assert (got - want).abs().max() <= want.abs().max() * 2.0 ** -18
 
 
+@pytest.mark.parametrize("gated,rot", [(0, 0), (0, 8), (1, 0)])
+def test_a_workspace_and_more_segments_than_a_grid_dimension_has(gated, rot):
+    """65536 segments of one token and one of 40: served with a workspace as without, and to the same bits"""
+    from mlx_vlm_amd import _lib, ops
+
+    g, n, D = torch.Generator().manual_seed(5), 65537, 8
+    T, C = n + 39, D + gated
+    q, k, v, gate = (torch.randn(T, D, generator=g).bfloat16().cuda() for _ in range(4))
+    pre, bias, decay = torch.randn(2, T, 1, generator=g).bfloat16().cuda(), torch.ones(1).bfloat16().cuda(), torch.tensor([0.9]).cuda()
+    inv = torch.tensor([1.0, 0.1, 0.01, 0.001]).cuda()
+    cu = torch.cat([torch.arange(n, dtype=torch.int32), torch.tensor([T], dtype=torch.int32)]).cuda()
+    slots, pos0 = torch.arange(n, dtype=torch.int32).cuda(), torch.zeros(n, dtype=torch.int32).cuda()
+
+    def run(ws):
+        state, ms, mtok, mprev = torch.zeros(n, 1, D, C, device="cuda"), torch.zeros(n, 1, device="cuda"), torch.zeros(T, 1, device="cuda"), torch.zeros(n, 1, device="cuda")
+        raw, out = torch.empty(T, 1, C, device="cuda"), torch.empty(T, D, dtype=torch.bfloat16, device="cuda")
+        a = _lib.RecurrenceArgs()
+        a.q, a.k, a.v, a.g, a.ldq, a.ldk, a.ldv, a.ldg, a.ldo = q.data_ptr(), k.data_ptr(), v.data_ptr(), gate.data_ptr(), D, D, D, D, D
+        a.qscale, a.kscale, a.eps, a.gate_act, a.gated, a.rot_dims, a.decay, a.inv_freq = 0.5, 0.25, 1e-5, 1, gated, rot, decay.data_ptr(), inv.data_ptr()
+        a.ipre, a.fpre, a.ldi, a.ldf, a.ib, a.fb, a.cap = pre[0].data_ptr(), pre[1].data_ptr(), 1, 1, bias.data_ptr(), bias.data_ptr(), 12.0
+        a.mstate, a.mtok, a.mprev = ms.data_ptr(), mtok.data_ptr(), mprev.data_ptr()
+        a.seg_start, a.seg_slot, a.seg_pos0 = cu.data_ptr(), slots.data_ptr(), pos0.data_ptr()
+        a.state, a.raw, a.out, a.H, a.D, a.Dv = state.data_ptr(), raw.data_ptr(), out.data_ptr(), 1, D, D
+        if ws is not None:
+            a.ws, a.ws_floats = ws.data_ptr(), ws.numel()
+        ops.linear_recurrence(a, n, T, False)
+        torch.cuda.synchronize()
+        return raw, state, ms
+
+    assert all(torch.equal(x, y) for x, y in zip(run(torch.empty(1 << 22, device="cuda")), run(None)))
+
+
 @pytest.mark.parametrize("gated,rot", [(0, 0), (0, 20), (1, 0)])
 def test_values_that_are_not_finite_stay_with_later_tokens(gated, rot):
     """an infinity and a NaN among the values of a prompt: the read-outs of the tokens before them, and of the columns beside them, are what they are without
