@@ -350,7 +350,7 @@ __global__ __launch_bounds__(256) void scaled_add_rms_kernel(AddRms p) {
 }
 
 // rows that do not come in pieces of four elements, or are wider than the registers
-template <typename T, typename HT>
+template <typename T, typename HT, bool SLOTS>
 __global__ __launch_bounds__(256) void scaled_add_rms_any_kernel(AddRms p) {
   __shared__ float red[4];
   const long t = blockIdx.x;
@@ -359,12 +359,13 @@ __global__ __launch_bounds__(256) void scaled_add_rms_any_kernel(AddRms p) {
   float q = 0.f;
   for (int d = threadIdx.x; d < p.D; d += 256) {        // (every lane re-reads only the entries it wrote)
     float v = xr[d];
-    if (y || p.slots) {
+    if (y || SLOTS) {
       float a = y ? ld_f(y + t * p.ldy + d) : 0.f;
-      for (int k = 0; k < p.nslots; ++k) {
-        const int s = p.slots[t * p.nslots + k];
-        if (s >= 0) a += p.rows32[(long)s * p.ldr + d];
-      }
+      if constexpr (SLOTS)
+        for (int k = 0; k < p.nslots; ++k) {
+          const int s = p.slots[t * p.nslots + k];
+          if (s >= 0) a += p.rows32[(long)s * p.ldr + d];
+        }
       v = fmaf(p.mult, a, v);
       if (y2) v = fmaf(p.mult2, ld_f(y2 + t * p.ldy2 + d), v);
       xr[d] = v;
@@ -383,7 +384,8 @@ int add_rms_launch(const AddRms& a, int rows, hipStream_t st) {
   const bool vec = a.D % 4 == 0 && n <= 16 && p16 % 16 == 0 && pt % (4 * sizeof(T)) == 0 && (uintptr_t)a.h % (4 * sizeof(HT)) == 0 &&
                    (!a.y || a.ldy % 4 == 0) && (!a.y2 || a.ldy2 % 4 == 0) && (!a.w || a.ldh % 4 == 0) && (!a.slots || a.ldr % 4 == 0);
 #define GO(N) hipLaunchKernelGGL((scaled_add_rms_kernel<T, HT, 4, N>), dim3(rows), dim3(256), 0, st, a)
-  if (!vec) hipLaunchKernelGGL((scaled_add_rms_any_kernel<T, HT>), dim3(rows), dim3(256), 0, st, a);
+  if (!vec && a.slots) hipLaunchKernelGGL((scaled_add_rms_any_kernel<T, HT, true>), dim3(rows), dim3(256), 0, st, a);
+  else if (!vec) hipLaunchKernelGGL((scaled_add_rms_any_kernel<T, HT, false>), dim3(rows), dim3(256), 0, st, a);
   else if (n <= 1) GO(1); else if (n <= 2) GO(2); else if (n <= 4) GO(4); else if (n <= 8) GO(8); else GO(16);
 #undef GO
   VLM_CHECK_LAUNCH();
