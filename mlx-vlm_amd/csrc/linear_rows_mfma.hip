@@ -133,11 +133,12 @@ __global__ __launch_bounds__(256) void linear_rows_mfma_kernel(RowsArgs p) {
 // R and NT (microseconds inside a graph, N x K, 8 bf16 rows): 1536 x 1536 R 6 NT 1 4.5, R 16 NT 1 8; 3584 x 3584 R 14 NT 1 8.8; from 4096 columns
 // on two tiles a wave share the activations: 4616 x 1536 R 10 NT 2 6.1, R 16 NT 1 7.6; 4608 x 3584 10.5 and 12.2.  Eight or sixteen waves instead
 // of four: 1536 x 8960 13.1 and 14.5 instead of 11.8.
+// Maps: as many workgroups a map as leave no compute unit two of them (us, 16 rows, 12 maps
+// [512, 128]: 264 workgroups of R 12 4.4, 240 of R 13 3.6; 9 rows, 28 maps [256, 192]: 308 of R 12 5.4, 252 of R 15 3.9).
 template <typename TA, typename TC>
 void launch_rows(RowsArgs a, int batch, hipStream_t st) {
-  const long all = (long)a.N * batch;
-  const int nt = all <= 4096 ? 1 : 2;
-  a.R = (int)std::min<long>(16, (all + 256 * nt - 1) / (256 * nt));
+  const int nt = (long)a.N * batch <= 4096 ? 1 : 2, per = std::max(1, 256 / batch) * nt;
+  a.R = std::min(16, (a.N + per - 1) / per);
   const dim3 grid((a.N + a.R * nt - 1) / (a.R * nt), batch), block(256);
   constexpr bool f = sizeof(TA) == 4;
   if constexpr (!f && sizeof(TC) == 4)
@@ -166,6 +167,9 @@ VLM_INTERNAL int vlm_linear_rows_mfma_try(const void* A, const void* W, void* C,
   // over workgroups (1536 x 8960, 16 rows: 12.6 and 15.2); many narrow maps of up to 8 rows are cheap here (28 of [512, 128]: 12.9 -> 4.6)
   // fp32 sums onto a stream keep the long K here up to 8 rows: the split form hands over bf16 (1536 x 21696, 2 / 4 / 8 rows: 26 / 26 / 32; vlm_linear_rows_bf16w
   // 48 / 76 / 140)
+  // two or three fp32 rows over a short K are cheaper a wave a column (2 rows, [2048, K], K = 64 / 256 / 384: 3.1 / 3.7 / 4.2, here 3.5 / 3.9 / 3.8; 3 rows,
+  // [1024, 64]: 3.3, 3.7)
+  if (a_f32 && (M == 2 ? K <= 256 : M == 3 && K <= 64)) return -1;
   const int va = a_f32 ? 4 : 8;
   // more rows over few columns, as blocks of 16: router logits [8, 1536] of 2048 rows 29 -> 7.5 us
   if (M > 32 ? N > 64 || batch > 1 || M > 65535 * 16 : false) return -1;
