@@ -663,8 +663,8 @@ int launch(const void* A, const void* W, void* C, int M, int N, int K, long lda,
   // token's result is the same bits in a prompt, in a portion and decoded alone
   constexpr bool all_f32 = sizeof(TA) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4;
   if constexpr (sizeof(TW) == 2) {
-    // a few rows (inside a graph, us): 12 maps [512, 128] to fp32, 8 rows 7.8 -> 3.9; 12 maps [128, 512] of fp32 rows, 2 / 8 / 16 rows 5.3 / 10.9 / 6.3 ->
-    // 4.8 / 5.3 / 6.3, one row 4.3 -> 4.8; [8, 1536] to fp32, 9 / 32 rows 12.3 / 15.6 -> 3.9 / 5.1.  Up to 8 fp32 rows with fp32 results stay on the
+    // a few rows (inside a graph, us): 12 maps [512, 128] to fp32, 8 rows 7.8 -> 3.9; 12 maps [128, 512] of fp32 rows, 2 / 3 / 16 rows 5.6 / 6.4 / 6.3 ->
+    // 4.2 / 4.3 / 5.2, one row 4.3 -> 4.8; [8, 1536] to fp32, 9 / 32 rows 12.3 / 15.6 -> 3.9 / 5.1.  Up to 8 fp32 rows with fp32 results stay on the
     // kernel below, whose sums are a little closer (relative error 7.5e-8 and 8.8e-8 at K = 200).
     if (M >= 2 && !(sizeof(TA) == 4 && sizeof(TC) == 4 && M <= 8)) {
       const int rc = vlm_linear_rows_mfma_try(A, W, C, M, N, K, lda, ldw, ldc, sizeof(TA) == 4, sizeof(TC) == 4, batch, sA, sW, sC, accumulate, st);
