@@ -239,7 +239,7 @@ int run(const vlm_recurrence_args& a, int nseg, int ntok, hipStream_t st) {
   int max_len = 0x7fffffff;
   const int longest = ntok - nseg + 1;                   // no segment of the step is longer (every segment has a token)
   // (the chunks' scan has the segments in a grid's second dimension)
-  if (!rowgate && !(gated && a.rot_dims) && a.ws && nseg <= 65535 && longest >= VLM_CHUNK_MIN && a.ws_floats - vlm_chunk_prep_floats(&a, ntok) >= (long)a.H * a.D * C) {
+  if (!rowgate && !(gated && a.rot_dims) && a.ws && nseg <= 65535 && longest >= vlm_chunk_from(&a) && a.ws_floats - vlm_chunk_prep_floats(&a, ntok) >= (long)a.H * a.D * C) {
     max_len = VLM_CHUNK_MIN - 1;
     const int rc = vlm_chunk_recurrence(&a, nseg, ntok, max_len, sizeof(T) == 4, st);
     if (rc) return rc;

@@ -124,9 +124,11 @@ class LanguageModel(RaggedLanguageModel):
     def _workspace(self, pl):
         """room for the chunk-parallel recurrences of a step with prompt portions, one piece for all layers (they follow each other on the stream): 2 H D fp32
         values a token (rotated q and k) or 4 H (gates), and H D columns per chunk of 64 tokens, the latter up to 256 MB (longer prompts run in windows of
-        chunks).  float32 serving stays token by token: the same bits however a prompt is cut"""
-        layers = [ns for ns in self._L if ns.type in ("retention", "mlstm")]
-        if pl.Tn - pl.nseg < 16 or not layers or self.dtype == torch.float32:             # (decode rows and short portions only)
+        chunks).  float32 serving stays token by token: the same bits however a prompt is cut; so do decode rows and portions that are faster so"""
+        if pl.Tn - pl.nseg < 16 or self.dtype == torch.float32:
+            return None
+        layers = [ns for ns in self._L if self._in_chunks(ns, pl)]
+        if not layers:
             return None
         chunks, need = pl.Tn // 64 + pl.nseg, 0
         for ns in layers:
@@ -134,6 +136,12 @@ class LanguageModel(RaggedLanguageModel):
             entries, per_token = ns.H * ns.D * (ns.Dv + gated), 4 * ns.H if gated else 2 * ns.H * ns.D if ns.rot_dims else 0
             need = max(need, per_token * pl.Tn + 4 + min(chunks, max(1, (64 << 20) // entries)) * entries)
         return torch.empty(need, dtype=torch.float32, device=self.device)
+
+    def _in_chunks(self, ns, pl):
+        if ns.type not in ("retention", "mlstm"):
+            return False
+        gated = ns.type == "mlstm"
+        return not gated and not ns.rot_dims or ops.recurrence_in_chunks(pl.lens, ns.H, ns.D, ns.Dv, gated)
 
     def _experts_grouped(self, ns, h):
         """whether a step's experts are evaluated pair by pair (the shared feed-forward as one more expert, which every token takes)"""
@@ -190,7 +198,7 @@ class LanguageModel(RaggedLanguageModel):
                 a.seg_start, a.seg_slot, a.seg_pos0 = cu_d.data_ptr(), slot_d.data_ptr(), pos0_d.data_ptr()
                 a.state, a.raw, a.out, a.ldo = pool.state[i].data_ptr(), raw.data_ptr(), cat.data_ptr(), cat.stride(0)
                 a.H, a.D, a.Dv, a.gated = ns.H, ns.D, ns.Dv, int(gated)
-                if ws is not None:
+                if ws is not None and self._in_chunks(ns, pl):
                     a.ws, a.ws_floats = ws.data_ptr(), ws.numel()
                 ops.linear_recurrence(a, nseg, Tn, is32)
                 keep.append(raw)

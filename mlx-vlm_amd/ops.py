@@ -651,6 +651,19 @@ def gelu_tanh_gate_rows(g, table, ids, col0, out=None):
     return out
 
 
+def recurrence_in_chunks(lens, H, D, Dv, gated):
+    """whether segments of these lengths are faster in chunks (a workspace in vlm_recurrence_args) than token by token: rotated fixed decay, or gated heads.  By
+    tokens the longest segment's chain or, with many of them, the work sets the time; in chunks a row of launches and the chunks' work.  us, by tokens |
+    in chunks, 12 heads of 128: 1 x 64 55 | 56, 1 x 100 81 | 57, 4 x 64 56 | 66, 12 x 40 44 | 78, 24 x 33 53 | 108; 28 heads: 1 x 200 155 | 75, 12 x 100 129 | 157, 24 x 33 97 | 177;
+    28 heads of 256: 1 x 100 92 | 110, 1 x 200 195 | 126"""
+    if max(lens) < (40 if D <= 64 else 72 if D <= 128 else 100):         # (vlm_chunk_from of csrc/chunk_recurrence.hpp)
+        return False
+    size, (chain, work) = H * D * Dv / 16384, (0.77, 4e-3) if D <= 128 else (0.9, 2.8e-3)
+    tokens = lambda some: max(chain * max(some), work * sum(some) * size) if some else 0      # noqa: E731
+    chunks = 29 + 0.21 * D + size * sum(0.24 + 0.08 * -(-n // 64) for n in lens if n > 16) + 5 * bool(gated)
+    return chunks + tokens([n for n in lens if n <= 16]) < 10 + tokens(lens)
+
+
 def linear_recurrence(args: "_lib.RecurrenceArgs", nseg: int, ntok: int, dtype_f32: bool):
     check(_lib.lib().vlm_linear_recurrence(C.byref(args), int(nseg), int(ntok), int(bool(dtype_f32)), _stream()), "linear_recurrence")
 

@@ -92,3 +92,13 @@ def test_oracle_is_consistent_under_cuts():
         y = f(x, pos, 6, 100.0)
         assert torch.allclose(y.norm(dim=-1), x.norm(dim=-1)) and torch.equal(y[0], x[0]) and torch.equal(y[..., 6:], x[..., 6:])
     assert not torch.allclose(O.rope_half(x, pos, 6, 100.0), O.rope_interleaved(x, pos, 6, 100.0))
+
+
+@pytest.mark.parametrize("lens,H,D,gated,chunks", [
+    ([20], 12, 128, False, False), ([18] * 32, 12, 128, False, False), ([18] * 32, 28, 256, True, False), ([64], 12, 128, True, False), ([71], 12, 128, False, False),
+    ([100], 12, 128, False, True), ([100], 28, 128, True, True), ([100], 28, 256, False, False), ([200], 28, 256, False, True), ([39], 12, 64, True, False),
+    ([64], 28, 64, False, True), ([100, 9, 30], 12, 128, False, True), ([300] + [1] * 8, 28, 128, True, True), ([120] * 4, 28, 256, False, False), ([100] * 12, 28, 128, True, False), ([200] * 8, 28, 128, True, True), ([150], 28, 256, True, True), ([300, 200, 40], 28, 256, False, True), ([33] * 24, 28, 128, False, False), ([2048], 12, 128, True, True)])
+def test_recurrences_of_short_portions_stay_token_by_token(lens, H, D, gated, chunks):
+    from mlx_vlm_amd import ops
+
+    assert ops.recurrence_in_chunks(lens, H, D, D, gated) is chunks
